@@ -136,80 +136,8 @@ static int adjoint_launch(int64_t count, const int32_t* n, const int32_t* nrhs, 
 // Factor every A[i] in place: systems with n <= TMVX_BATCH_NMAX through one
 // batched launch, larger ones through the blocked LU, one after another.
 // Medium systems (above the register-resident batched kernel's limit, up to
-// WG_NMAX): one 1024-thread workgroup factors one system in place, column
-// by column, in global memory (L2-resident at these sizes): TMV's pivot
-// rule (largest |a|, first row on ties), its underflow rule (the column is
-// zeroed from the diagonal down and interchanged with itself), the column
-// scaled by the pivot's reciprocal, then the rank-1 update of the trailing
-// matrix spread over all threads.  info[sys] = 1-based first zero pivot.
+// WG_NMAX) in one launch of a workgroup per system (tmvx_lu_wg.hip).
 constexpr int WG_NMAX = 1024;
-
-template <typename T>
-__global__ void __launch_bounds__(1024)
-lu_wg_kernel(const int* __restrict__ order, const int32_t* __restrict__ nv, T* const* A,
-             int64_t* const* piv, int32_t* __restrict__ info)
-{
-    constexpr int NW = 1024 / 64;
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    __shared__ T s_v[NW];
-    __shared__ int s_i[NW];
-    __shared__ int s_p, s_zero;
-    __shared__ T s_inv;
-    const int sys = order[blockIdx.x];
-    const int n = nv[sys];
-    T* a = A[sys];
-    int64_t* pv = piv[sys];
-    int first_zero = 0;
-    for (int j = 0; j < n; ++j) {
-        T bv = T(-1);
-        int bi = INT_MAX;
-        for (int i = j + t; i < n; i += 1024) {
-            const T v = fabs(a[i + (i64)j * n]);
-            if (v > bv) { bv = v; bi = i; }
-        }
-        wave_argmax(bv, bi);
-        if (lane == 0) { s_v[wave] = bv; s_i[wave] = bi; }
-        __syncthreads();
-        if (t == 0) {
-            T v = s_v[0];
-            int ii = s_i[0];
-            for (int q = 1; q < NW; ++q)
-                if (better(s_v[q], s_i[q], v, ii)) { v = s_v[q]; ii = s_i[q]; }
-            const bool zero = !(v >= tiny<T>());
-            s_zero = zero ? 1 : 0;
-            s_p = zero ? j : ii;
-            pv[j] = zero ? j : ii;
-            if (zero && first_zero == 0) first_zero = j + 1;
-        }
-        __syncthreads();
-        if (s_zero) {
-            for (int i = j + t; i < n; i += 1024) a[i + (i64)j * n] = T(0);
-            __syncthreads();
-            continue;
-        }
-        const int p = s_p;
-        if (p != j)
-            for (int c = t; c < n; c += 1024) {
-                const T x = a[j + (i64)c * n];
-                a[j + (i64)c * n] = a[p + (i64)c * n];
-                a[p + (i64)c * n] = x;
-            }
-        __syncthreads();
-        if (t == 0) s_inv = T(1) / a[j + (i64)j * n];
-        __syncthreads();
-        const T inv = s_inv;
-        for (int i = j + 1 + t; i < n; i += 1024) a[i + (i64)j * n] *= inv;
-        __syncthreads();
-        const int m = n - j - 1;
-        const i64 tot = (i64)m * m;
-        for (i64 e = t; e < tot; e += 1024) {
-            const int i = j + 1 + (int)(e % m), c = j + 1 + (int)(e / m);
-            a[i + (i64)c * n] -= a[i + (i64)j * n] * a[j + (i64)c * n];
-        }
-        __syncthreads();
-    }
-    if (t == 0) info[sys] = first_zero;
-}
 
 template <typename T>
 static int getrf_batched_impl(int64_t count, const int32_t* n_host, T* const* A, int64_t* const* piv,
@@ -243,9 +171,9 @@ static int getrf_batched_impl(int64_t count, const int32_t* n_host, T* const* A,
                             s) != hipSuccess))
             rc = TMVX_ERR_HIP;
         if (rc == TMVX_OK) {
-            hipLaunchKernelGGL(lu_wg_kernel<T>, dim3((unsigned)medium.size()), dim3(1024), 0, s,
-                               (const int*)dord, (const int32_t*)dn, A, piv, info);
-            rc = hip_status(hipGetLastError());
+            int nmax = 0;
+            for (int i : medium) nmax = std::max(nmax, (int)n_host[i]);
+            rc = lu_wg_launch<T>(nmax, (int)medium.size(), dord, dn, A, piv, info, s);
         }
         if (hipStreamSynchronize(s) != hipSuccess && rc == TMVX_OK) rc = TMVX_ERR_HIP;
         hipFree(dord);

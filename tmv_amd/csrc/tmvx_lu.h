@@ -85,6 +85,13 @@ template <typename T>
 int getrs_perm(int trans, i64 n, i64 nrhs, const T* LU, i64 lda, const i64* perm, T* B,
                i64 ldb, int* d_singular, hipStream_t s, int inv = 0);
 
+// One workgroup per system factors systems order[0..count) of a batch in
+// place, orders n[order[i]] <= nmax <= 1024 (tmvx_lu_wg.hip); n, order, the
+// pointer arrays and info (1-based first zero pivot or 0) on the device.
+template <typename T>
+int lu_wg_launch(int nmax, int count, const int* d_order, const int32_t* d_n, T* const* A,
+                 int64_t* const* piv, int32_t* info, hipStream_t s);
+
 // A side stream with two events for the look-ahead factorisation, taken
 // from a per-device pool (tmvx_util.hip) and returned after use; idle sets
 // have no pending work.

@@ -57,7 +57,7 @@ __device__ __forceinline__ void wave_argmax(T& v, int& i)
 // stage, then a ballot of the lanes holding it; only an exact tie takes a
 // second reduction, the minimum index among the tied lanes.  NaN values
 // never win (fmax ignores them); with no comparable value the result is
-// (-1, INT_MAX).  NL = 64 reduces the wave, NL = 8 lanes 0..7.
+// (-1, INT_MAX).  NL = 64 reduces the wave, NL = 8 / 16 lanes 0..NL-1.
 template <int CTRL, int RM, typename T>
 __device__ __forceinline__ T dpp_max_step(T v)
 {
@@ -81,7 +81,7 @@ __device__ __forceinline__ int dpp_min_step(int i)
 template <int NL, typename T>
 __device__ __forceinline__ void lanes_argmax(T v, int i, T& bv, int& bi)
 {
-    static_assert(NL == 64 || NL == 8, "64 or 8 lanes");
+    static_assert(NL == 64 || NL == 16 || NL == 8, "64, 16 or 8 lanes");
     const int lane = threadIdx.x & 63;
     T m = v;
     m = dpp_max_step<0xB1, 0xf>(m);      // quad_perm [1,0,3,2]
@@ -93,6 +93,7 @@ __device__ __forceinline__ void lanes_argmax(T v, int i, T& bv, int& bi)
         m = dpp_max_step<0x143, 0xc>(m); // row_bcast:31
         m = readlane(m, 63);
     } else {
+        if constexpr (NL == 16) m = dpp_max_step<0x140, 0xf>(m);
         m = readlane(m, 0);
     }
     const bool in = NL == 64 || lane < NL;
@@ -113,6 +114,7 @@ __device__ __forceinline__ void lanes_argmax(T v, int i, T& bv, int& bi)
         x = dpp_min_step<0x143, 0xc>(x);
         bi = __builtin_amdgcn_readlane(x, 63);
     } else {
+        if constexpr (NL == 16) x = dpp_min_step<0x140, 0xf>(x);
         bi = __builtin_amdgcn_readlane(x, 0);
     }
 }
