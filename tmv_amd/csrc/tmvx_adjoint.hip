@@ -9,16 +9,15 @@
 // (x % A, src/TMV_LUDiv.cpp:369-410) and the rank-k update its MultMM
 // (src/TMV_MultMM.cpp:404-477).
 //
-// Batched kernels: one wave per system solves A^T gB = G column by column
-// with the stored factors (dot-product sweeps over contiguous columns of U
-// and L); then many workgroups per system write gradA as
+// Batched kernels: a workgroup or a wave per system solves A^T gB = G with the stored factors; then many workgroups per system write
+// gradA as
 // -sum_c gB(:,c) X(k,c), 16 columns each (gradA, the n^2 output, is
 // written once and read only when accumulating).  The recompute variant
 // factors copies of the original matrices first, for callers that did not
 // keep the factors.
 #include "tmvx_lu.h"
 #include "tmvx_pivot.h"
-#include "tmvx_wave_solve.h"
+#include "tmvx_wg_solve.h"
 #include "../../include/tmvx_batched.h"
 
 #include <algorithm>
@@ -29,9 +28,21 @@ namespace tmvx {
 
 constexpr int ADJ_RHS = 4;     // right-hand sides held in registers at once
 
+// gradB = A^-T G, a workgroup (n <= 64: a wave) per system, or, for more
+// than WS_WG_MAX systems, one wave per system.
+template <typename T>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+adjoint_batched_kernel(int count, const int* __restrict__ nv, const int* __restrict__ nrhsv,
+                       const T* const* __restrict__ LUv, const i64* const* __restrict__ pivv,
+                       const T* const* Gv, T* const* gBv)
+{
+    __shared__ WgSolveShared<T> sh;
+    wg_getrs_batch<T, true>(count, nv, nrhsv, LUv, pivv, Gv, gBv, sh);
+}
+
 template <typename T>
 __global__ void __launch_bounds__(64)
-adjoint_batched_kernel(int count, const int* __restrict__ nv, const int* __restrict__ nrhsv,
+adjoint_wave_kernel(int count, const int* __restrict__ nv, const int* __restrict__ nrhsv,
                        const T* const* __restrict__ LUv, const i64* const* __restrict__ pivv,
                        const T* const* __restrict__ Gv, T* const* __restrict__ gBv)
 {
@@ -55,9 +66,7 @@ adjoint_batched_kernel(int count, const int* __restrict__ nv, const int* __restr
     }
 }
 
-// gradA (+)= -gradB X^T for the systems the wave solves handled, spread
-// over many workgroups (one wave per system writing its n^2 gradient left
-// most of HBM idle): workgroup item (sys, kb) forms columns
+// gradA (+)= -gradB X^T, spread over many workgroups: workgroup item (sys, kb) forms columns
 // [ADJ_KC kb, ADJ_KC kb + ADJ_KC) of gradA, one row per thread.  The
 // right-hand sides are taken in blocks of ADJ_RHS, the first block's sum
 // written (or added, when accumulating) and each later block's added, in
@@ -124,8 +133,12 @@ static int adjoint_launch(int64_t count, const int32_t* n, const int32_t* nrhs, 
     if (count == 0) return TMVX_OK;
     if (!n || !nrhs || !LU || !piv || !X || !G || !gB || !gA) return TMVX_ERR_ARG;
     const unsigned grid = (unsigned)std::min<int64_t>(count, 4096);
-    hipLaunchKernelGGL(adjoint_batched_kernel<T>, dim3(grid), dim3(64), 0, s, (int)count, n, nrhs,
-                       LU, (const i64* const*)piv, G, gB);
+    if (count > WS_WG_MAX)
+        hipLaunchKernelGGL(adjoint_wave_kernel<T>, dim3(grid), dim3(64), 0, s, (int)count, n, nrhs,
+                           LU, (const i64* const*)piv, G, gB);
+    else
+        hipLaunchKernelGGL(adjoint_batched_kernel<T>, dim3(grid), dim3(256), 0, s, (int)count, n,
+                           nrhs, LU, (const i64* const*)piv, G, gB);
     TMVX_TRY(hip_status(hipGetLastError()));
     const unsigned grid2 = (unsigned)std::min<int64_t>(count * (WS_NMAX / ADJ_KC), 16384);
     hipLaunchKernelGGL(adjoint_grad_kernel<T>, dim3(grid2), dim3(256), 0, s, (int)count, n, nrhs,

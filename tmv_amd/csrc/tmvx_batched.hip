@@ -34,7 +34,7 @@
 // captured in a hipGraph and replayed.
 #include "tmvx_lu.h"
 #include "tmvx_pivot.h"
-#include "tmvx_wave_solve.h"
+#include "tmvx_wg_solve.h"
 #include "../../include/tmvx_batched.h"
 
 #include <algorithm>
@@ -61,18 +61,6 @@ struct BLds {
     T mult[NMAX];           // multipliers, indexed by row
     int pos[NMAX];          // final position of each row
     int piv[NMAX];          // interchange list, written out at the end
-};
-
-struct GroupSync {
-    __device__ __forceinline__ void operator()() const { __syncthreads(); }
-};
-struct WaveSync {
-    __device__ __forceinline__ void operator()() const
-    {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    }
 };
 
 template <typename T>
@@ -362,11 +350,22 @@ batched_lu_solve_kernel(BatchArgs<T> args)
 }
 
 // ---------------------------------------------------------------------------
-// Batched solve with stored factors: one wave per (system, right-hand side).
+// Batched solve with stored factors: a workgroup (n <= 64: a wave) per
+// system, or, for more than WS_WG_MAX systems, one wave per system.
 // ---------------------------------------------------------------------------
+template <typename T, bool TRANS>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+batched_getrs_kernel(int count, const int* __restrict__ nv, const int* __restrict__ nrhsv,
+                     const T* const* __restrict__ LUv, const i64* const* __restrict__ pivv,
+                     T* const* Bv)
+{
+    __shared__ WgSolveShared<T> sh;
+    wg_getrs_batch<T, TRANS>(count, nv, nrhsv, LUv, pivv, (const T* const*)Bv, Bv, sh);
+}
+
 template <typename T>
 __global__ void __launch_bounds__(256)
-batched_getrs_kernel(int trans, int count, const int* __restrict__ nv,
+batched_getrs_wave_kernel(int trans, int count, const int* __restrict__ nv,
                      const int* __restrict__ nrhsv, const T* const* __restrict__ LUv,
                      const i64* const* __restrict__ pivv, T* const* __restrict__ Bv)
 {
@@ -821,22 +820,24 @@ int tmvx_gesv_batched_f32(tmvx_batch_plan p, float* const* A, int64_t* const* pi
     return batch_launch<float>(p, A, (i64* const*)piv, B, info, (hipStream_t)stream);
 }
 
+extern "C++" template <typename T>
 static int getrs_batched_launch(int trans, int64_t count, const int32_t* n, const int32_t* nrhs,
-                                const void* LU, const int64_t* const* piv, void* B, int f64,
+                                const T* const* LU, const int64_t* const* piv, T* const* B,
                                 hipStream_t s)
 {
     if (count < 0 || count > INT_MAX) return TMVX_ERR_ARG;
     if (count == 0) return TMVX_OK;
     if (!n || !nrhs || !LU || !piv || !B) return TMVX_ERR_ARG;
-    const unsigned grid = 2048;      // 8192 waves; wave w takes systems w, w + 8192, ...
-    if (f64)
-        hipLaunchKernelGGL(batched_getrs_kernel<double>, dim3(grid), dim3(256), 0, s, trans,
-                           (int)count, n, nrhs, (const double* const*)LU, (const i64* const*)piv,
-                           (double* const*)B);
+    const dim3 grid((unsigned)std::min<int64_t>(count, 2048)), block(256);
+    if (count > WS_WG_MAX)           // 8192 waves; wave w takes systems w, w + 8192, ...
+        hipLaunchKernelGGL(batched_getrs_wave_kernel<T>, dim3(2048), block, 0, s, trans,
+                           (int)count, n, nrhs, LU, (const i64* const*)piv, B);
+    else if (trans)
+        hipLaunchKernelGGL((batched_getrs_kernel<T, true>), grid, block, 0, s, (int)count, n, nrhs,
+                           LU, (const i64* const*)piv, B);
     else
-        hipLaunchKernelGGL(batched_getrs_kernel<float>, dim3(grid), dim3(256), 0, s, trans,
-                           (int)count, n, nrhs, (const float* const*)LU, (const i64* const*)piv,
-                           (float* const*)B);
+        hipLaunchKernelGGL((batched_getrs_kernel<T, false>), grid, block, 0, s, (int)count, n, nrhs,
+                           LU, (const i64* const*)piv, B);
     return hip_status(hipGetLastError());
 }
 
@@ -844,14 +845,14 @@ int tmvx_getrs_batched_f64(int trans, int64_t count, const int32_t* n, const int
                            const double* const* LU, const int64_t* const* piv, double* const* B,
                            void* stream)
 {
-    return getrs_batched_launch(trans, count, n, nrhs, LU, piv, (void*)B, 1, (hipStream_t)stream);
+    return getrs_batched_launch<double>(trans, count, n, nrhs, LU, piv, B, (hipStream_t)stream);
 }
 
 int tmvx_getrs_batched_f32(int trans, int64_t count, const int32_t* n, const int32_t* nrhs,
                            const float* const* LU, const int64_t* const* piv, float* const* B,
                            void* stream)
 {
-    return getrs_batched_launch(trans, count, n, nrhs, LU, piv, (void*)B, 0, (hipStream_t)stream);
+    return getrs_batched_launch<float>(trans, count, n, nrhs, LU, piv, B, (hipStream_t)stream);
 }
 
 int tmvx_gemm_batched_f64(int64_t count, const int32_t* m, const int32_t* n, const int32_t* k,

@@ -13,18 +13,24 @@
 //     row's position); per column each wave's best row writes itself to LDS
 //     before the column's only barrier, then every wave picks the winner
 //     among the waves' candidates and updates its rows;
-//   interchanges + U12 = L11^-1 A12: one column per lane, the 32 rows in
+//   U12 = L11^-1 A12: one column per lane, its 32 pivot rows gathered into
 //     registers, L11 read from LDS as broadcasts; U12 stays in LDS;
 //   A22 -= L21 U12 on MFMA, 32 x 32 of A22 per wave, L21 read from L2, U12
-//     from LDS.  The product is formed transposed, so that the 16 lanes of
+//     from LDS; the interchanges are the row each update is read from.  The product is formed transposed, so that the 16 lanes of
 //     an MFMA column hold 16 consecutive rows: A22 moves in 128-byte runs.
 // The interchanges of the columns left of a panel (L's) are all applied at
 // the end, one pass over the matrix (thread per row, the source row traced
 // back through the interchange list), instead of a scattered pass per panel.
 //
-// Bound: the panel's chain of one barrier per column and the latency of
-// the A22 tiles, with two workgroups per CU to overlap them; n^3 / (3 WL_NB)
-// elements of A22 are read and written.
+// Bound: the panel's chain of one barrier per column (0.8 us a column with
+// two workgroups on the CU, most of it LDS traffic: every wave writes its
+// candidate row and reads the winner's) and the latency of the A22 tiles;
+// n^3 / (3 WL_NB) elements of A22 are read and written.  Measured, 512
+// systems of n = 256 FP64: 0.63 ms (panels 0.20-0.22, U12 0.10, A22 0.18,
+// L's interchanges 0.03), against 9.7 ms for rank-1 updates of the whole
+// matrix in global memory with six barriers a column; 0.87 ms with the pivot
+// search on floating-point maxima, a rotated panel row and the interchanges
+// as a pass of their own.
 #include "tmvx_lu.h"
 #include "tmvx_pivot.h"
 
@@ -48,19 +54,26 @@ lu_wg_kernel(const int* __restrict__ order, const int32_t* __restrict__ nv, T* c
     typedef typename Vec16<T>::type VT;
     typedef typename Mfma<T>::v4 v4;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    constexpr int NWP = NW <= 4 ? 4 : NW <= 8 ? 8 : 16;           // lanes that compare waves
     __shared__ __attribute__((aligned(16))) T s_row[2][NW][NB];   // the waves' candidate rows
-    __shared__ T s_v[2][NW];
-    __shared__ int s_i[2][NW];
+    __shared__ unsigned s_hi[2][16], s_lo[2][16];                 // their keys and positions
+    __shared__ int s_pos[2][16];
     __shared__ __attribute__((aligned(16))) T s_l[NB][NB];        // s_l[k][i] = L11(i, k)
     __shared__ __attribute__((aligned(16))) T s_u[NB][WL_LDU];    // U12 of one column chunk
-    __shared__ int s_src[NB];     // panel row k comes from panel-relative row s_src[k]
-    __shared__ int s_dst[NB];     // the row that was panel row k goes to s_dst[k]
-    __shared__ int s_piv[NTH];    // the whole interchange list
+    __shared__ short s_src[NB];   // panel row k comes from panel-relative row s_src[k]
+    __shared__ short s_from[NTH]; // row r of the panel's moved rows comes from s_from[r]
+    __shared__ short s_piv[NTH];  // the whole interchange list
     const int sys = order[blockIdx.x];
     const int n = nv[sys];
     T* __restrict__ A = Av[sys];
     const i64 ld = n;
     int first_zero = 0;
+    if (t < 16) {                       // no candidate from waves that do not exist
+        s_hi[0][t] = s_hi[1][t] = 0u;
+        s_lo[0][t] = s_lo[1][t] = 0u;
+        s_pos[0][t] = s_pos[1][t] = INT_MAX;
+    }
+    __syncthreads();
 
     for (int j = 0; j < n; j += NB) {
         const int m = n - j, jb = m < NB ? m : NB;
@@ -71,87 +84,68 @@ lu_wg_kernel(const int* __restrict__ order, const int32_t* __restrict__ nv, T* c
         for (int c = 0; c < NB; ++c) row[c] = (own && c < jb) ? A[(j + t) + (j + c) * ld] : T(0);
         int pos = t;
         bool used = !own;
-        // blocks of 8 columns, the block in hand in row[0..8): after block b
-        // the row is rotated by 8, row[c] is column 8 b + c while that is < NB
-        for (int b = 0; b < NB / 8; ++b) {
-            static_for<0, 8>([&](auto kc) __attribute__((always_inline)) {
-                constexpr int kk = decltype(kc)::value;
-                const int k = 8 * b + kk;
-                if (k >= jb) return;                                  // uniform
-                constexpr int par = kk & 1;
-                T v;
-                int vi;
-                lanes_argmax<64, T>(used ? T(-1) : T(fabs(row[kk])), pos, v, vi);
-                if (lane == 0) { s_v[par][wave] = v; s_i[par][wave] = vi; }
-                if (!used && pos == vi) {
-                    static_for<0, NB / VN>([&](auto qc) __attribute__((always_inline)) {
-                        constexpr int q = decltype(qc)::value * VN;
-                        if constexpr (q + VN > kk) {
-                            VT x;
-                            static_for<0, VN>([&](auto uc) __attribute__((always_inline)) {
-                                x[decltype(uc)::value] = row[q + decltype(uc)::value];
-                            });
-                            *reinterpret_cast<VT*>(&s_row[par][wave][q]) = x;
-                        }
+        // (a last panel narrower than NB runs its missing columns as zero
+        // columns, with nothing recorded)
+        static_for<0, NB>([&](auto kc) __attribute__((always_inline)) {
+            constexpr int k = decltype(kc)::value, par = k & 1;
+            const unsigned hi = used ? 0u : mag_hi(row[k]), lo = mag_lo(row[k]);
+            unsigned m;
+            const int wl = lanes_best<64, T>(hi, lo, pos, m);
+            if (lane == wl) {
+                s_hi[par][wave] = m;
+                s_lo[par][wave] = lo;
+                s_pos[par][wave] = pos;
+                static_for<k / VN, NB / VN>([&](auto qc) __attribute__((always_inline)) {
+                    constexpr int q = decltype(qc)::value * VN;
+                    VT x;
+                    static_for<0, VN>([&](auto uc) __attribute__((always_inline)) {
+                        x[decltype(uc)::value] = row[q + decltype(uc)::value];
                     });
-                }
-                __syncthreads();
-                T gv;
-                int gi;
-                const int ci = lane < NW ? s_i[par][lane] : INT_MAX;
-                lanes_argmax<(NW > 8 ? 16 : 8)>(lane < NW ? s_v[par][lane] : T(-1), ci, gv, gi);
-                const bool zero = !(gv >= tiny<T>());
-                if (t == 0) s_piv[j + k] = j + (zero ? k : gi);
-                if (zero) {
-                    if (first_zero == 0) first_zero = j + k + 1;
-                    if (!used) row[kk] = T(0);
-                    if (!used && pos == k) used = true;
-                } else {
-                    const unsigned long long hw = __ballot(lane < NW && ci == gi);
-                    const T* pr = &s_row[par][hw ? (int)__builtin_ctzll(hw) : 0][0];
-                    if (!used && pos == gi) { used = true; pos = k; }
-                    else if (!used && pos == k) pos = gi;
-                    // rows already pivotal take multiplier 0 for their
-                    // updates and keep their own column
-                    const T l = row[kk] * (T(1) / pr[kk]);
-                    if (!used) row[kk] = l;
-                    const T lu = used ? T(0) : l;
-                    static_for<0, NB / 8>([&](auto cc) __attribute__((always_inline)) {
-                        constexpr int c0 = decltype(cc)::value * 8;
-                        if (c0 >= NB - 8 * b) return;                 // uniform
-                        static_for<0, 8 / VN>([&](auto qc) __attribute__((always_inline)) {
-                            constexpr int q = c0 + decltype(qc)::value * VN;
-                            if constexpr (q + VN > kk + 1) {
-                                const VT u = *reinterpret_cast<const VT*>(pr + q);
-                                static_for<0, VN>([&](auto uc) __attribute__((always_inline)) {
-                                    constexpr int x = decltype(uc)::value;
-                                    if constexpr (q + x > kk)
-                                        if (!used) row[q + x] -= lu * u[x];
-                                });
-                            }
-                        });
-                    });
-                }
+                    *reinterpret_cast<VT*>(&s_row[par][wave][q]) = x;
+                });
+            }
+            __syncthreads();
+            unsigned gm;
+            const int cpos = s_pos[par][lane & 15];
+            const int ww = lanes_best<NWP, T>(s_hi[par][lane & 15], s_lo[par][lane & 15], cpos, gm);
+            const bool zero = gm < mag_tiny<T>();                      // TMV_Underflow
+            const int p = zero ? k : __builtin_amdgcn_readlane(cpos, ww);
+            const T* pr = &s_row[par][ww][0];
+            T u[NB];
+            static_for<k / VN, NB / VN>([&](auto qc) __attribute__((always_inline)) {
+                constexpr int q = decltype(qc)::value * VN;
+                const VT x = *reinterpret_cast<const VT*>(pr + q);
+                static_for<0, VN>([&](auto uc) __attribute__((always_inline)) {
+                    u[q + decltype(uc)::value] = x[decltype(uc)::value];
+                });
             });
-            T first[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) first[q] = row[q];
-#pragma unroll
-            for (int c = 0; c < NB - 8; ++c) row[c] = row[c + 8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) row[NB - 8 + q] = first[q];
-        }
+            if (t == 0 && k < jb) s_piv[j + k] = (short)(j + p);
+            if (zero && first_zero == 0 && k < jb) first_zero = j + k + 1;
+            if (zero && !used) row[k] = T(0);
+            const bool isp = !used && pos == p;
+            if (!used && pos == k) pos = p;
+            if (isp) pos = k;
+            used = used || isp;
+            const T l = row[k] * (T(1) / u[k]);
+            if (!used && !zero) {
+                row[k] = l;
+                static_for<k + 1, NB>([&](auto cc) __attribute__((always_inline)) {
+                    constexpr int c = decltype(cc)::value;
+                    row[c] -= l * u[c];
+                });
+            }
+        });
         // rows to their final positions; L11 and the row moves to LDS
         if (own) {
 #pragma unroll
             for (int c = 0; c < NB; ++c)
                 if (c < jb) A[(j + pos) + (j + c) * ld] = row[c];
             if (pos < NB) {
-                s_src[pos] = t;
+                s_src[pos] = (short)t;
 #pragma unroll
                 for (int c = 0; c < NB; ++c) s_l[c][pos] = row[c];
             }
-            if (t < NB) s_dst[t] = pos;
+            s_from[pos] = (short)t;
         }
         __syncthreads();
         if (m <= NB) break;
@@ -165,45 +159,40 @@ lu_wg_kernel(const int* __restrict__ order, const int32_t* __restrict__ nv, T* c
                     for (int k = 0; k < NB; ++k) s_u[k][c] = T(0);
                     continue;
                 }
-                T* __restrict__ col = A + j + (cb + c) * ld;
+                const T* __restrict__ col = A + j + (cb + c) * ld;
                 T x[NB];
 #pragma unroll
                 for (int k = 0; k < NB; ++k) x[k] = col[s_src[k]];
-                // every gathered row has been read before a row is moved
-                // over it; the panel's own rows are rewritten only below
-                __builtin_amdgcn_s_waitcnt(0);
-                static_for<0, NB / 8>([&](auto qc) __attribute__((always_inline)) {
-                    constexpr int k0 = decltype(qc)::value * 8;
-                    __asm__ volatile("" ::: "memory");
-                    T old[8];
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) old[k] = s_dst[k0 + k] >= NB ? col[k0 + k] : T(0);
-#pragma unroll
-                    for (int k = 0; k < 8; ++k)
-                        if (s_dst[k0 + k] >= NB) col[s_dst[k0 + k]] = old[k];
-                });
+                // (L11's column k is read when x[k - 4] is final: an opaque
+                // dependency, or the reads would be hoisted to the top)
+                int off = 0;
                 static_for<0, NB>([&](auto kc) __attribute__((always_inline)) {
                     constexpr int k = decltype(kc)::value;
+                    if constexpr (k >= 4 && k % 4 == 0) __asm__ volatile("" : "+v"(off) : "v"(x[k - 4]));
+                    const T* lk = &s_l[k][0] + off;
                     static_for<k + 1, NB>([&](auto ic) __attribute__((always_inline)) {
                         constexpr int i = decltype(ic)::value;
-                        x[i] -= s_l[k][i] * x[k];
+                        x[i] -= lk[i] * x[k];
                     });
-                    __asm__ volatile("" ::: "memory");   // L11's reads stay in their step
                 });
 #pragma unroll
-                for (int k = 0; k < NB; ++k) { col[k] = x[k]; s_u[k][c] = x[k]; }
+                for (int k = 0; k < NB; ++k) s_u[k][c] = x[k];
             }
             __syncthreads();
+            // A22: row r takes its update from the row that the interchanges
+            // bring to it (one of the panel's own rows, unless it stays), so
+            // the moves cost no pass of their own
             const int li = lane & 15, g = lane >> 4;
             const int tm = (m - NB + 31) / 32, tn = (nc + 31) / 32;
             for (int tile = wave; tile < tm * tn; tile += NW) {
-                const int r0 = j + NB + 32 * (tile % tm), c0 = 32 * (tile / tm);
-                int rr[2];                  // rows past the end read the last one
+                const int r0 = NB + 32 * (tile % tm), c0 = 32 * (tile / tm);
+                int rr[2], fr[2];           // rows past the end read the last one
                 T lf[2][8], uf[2][8];
                 static_for<0, 2>([&](auto ic) __attribute__((always_inline)) {
                     constexpr int i = decltype(ic)::value;
                     const int r = r0 + 16 * i + li;
-                    rr[i] = r < n ? r : n - 1;
+                    rr[i] = j + (r < m ? r : m - 1);
+                    fr[i] = j + s_from[r < m ? r : m - 1];
                 });
                 v4 acc[2][2];               // acc[jc][i]: columns c0 + 16 jc.., rows r0 + 16 i..
                 static_for<0, 2>([&](auto jc) __attribute__((always_inline)) {
@@ -212,7 +201,7 @@ lu_wg_kernel(const int* __restrict__ order, const int32_t* __restrict__ nv, T* c
                             constexpr int q = decltype(rc)::value;
                             const int c = c0 + 16 * decltype(jc)::value + Mfma<T>::row(g, q);
                             acc[decltype(jc)::value][decltype(ic)::value][q] =
-                                A[rr[decltype(ic)::value] + (cb + (c < nc ? c : nc - 1)) * ld];
+                                A[fr[decltype(ic)::value] + (cb + (c < nc ? c : nc - 1)) * ld];
                         });
                     });
                 });
@@ -238,12 +227,16 @@ lu_wg_kernel(const int* __restrict__ order, const int32_t* __restrict__ nv, T* c
                         static_for<0, 4>([&](auto rc) __attribute__((always_inline)) {
                             constexpr int q = decltype(rc)::value, i = decltype(ic)::value;
                             const int c = c0 + 16 * decltype(jc)::value + Mfma<T>::row(g, q);
-                            if (r0 + 16 * i + li < n && c < nc)
+                            if (r0 + 16 * i + li < m && c < nc)
                                 A[rr[i] + (cb + c) * ld] = acc[decltype(jc)::value][i][q];
                         });
                     });
                 });
             }
+            __syncthreads();
+            // U12 over the panel's old rows, which A22 has taken by now
+            for (int e = t; e < NB * nc; e += NTH)
+                A[j + (e & (NB - 1)) + (cb + e / NB) * ld] = s_u[e & (NB - 1)][e / NB];
             __syncthreads();
         }
     }

@@ -57,7 +57,7 @@ __device__ __forceinline__ void wave_argmax(T& v, int& i)
 // stage, then a ballot of the lanes holding it; only an exact tie takes a
 // second reduction, the minimum index among the tied lanes.  NaN values
 // never win (fmax ignores them); with no comparable value the result is
-// (-1, INT_MAX).  NL = 64 reduces the wave, NL = 8 / 16 lanes 0..NL-1.
+// (-1, INT_MAX).  NL = 64 reduces the wave, NL = 8 lanes 0..7.
 template <int CTRL, int RM, typename T>
 __device__ __forceinline__ T dpp_max_step(T v)
 {
@@ -81,7 +81,7 @@ __device__ __forceinline__ int dpp_min_step(int i)
 template <int NL, typename T>
 __device__ __forceinline__ void lanes_argmax(T v, int i, T& bv, int& bi)
 {
-    static_assert(NL == 64 || NL == 16 || NL == 8, "64, 16 or 8 lanes");
+    static_assert(NL == 64 || NL == 8, "64 or 8 lanes");
     const int lane = threadIdx.x & 63;
     T m = v;
     m = dpp_max_step<0xB1, 0xf>(m);      // quad_perm [1,0,3,2]
@@ -93,7 +93,6 @@ __device__ __forceinline__ void lanes_argmax(T v, int i, T& bv, int& bi)
         m = dpp_max_step<0x143, 0xc>(m); // row_bcast:31
         m = readlane(m, 63);
     } else {
-        if constexpr (NL == 16) m = dpp_max_step<0x140, 0xf>(m);
         m = readlane(m, 0);
     }
     const bool in = NL == 64 || lane < NL;
@@ -114,9 +113,75 @@ __device__ __forceinline__ void lanes_argmax(T v, int i, T& bv, int& bi)
         x = dpp_min_step<0x143, 0xc>(x);
         bi = __builtin_amdgcn_readlane(x, 63);
     } else {
-        if constexpr (NL == 16) x = dpp_min_step<0x140, 0xf>(x);
         bi = __builtin_amdgcn_readlane(x, 0);
     }
+}
+
+// Pivot search on integer keys.  |a| >= 0 orders as its bits do, so the
+// search runs on the high 32 bits alone (one v_max_u32 with DPP a stage,
+// where a double's maximum takes two moves and two v_max_f64); only lanes
+// that tie there compare the low words, then positions (TMV's tie rule).
+// Rows out of the search and NaN carry key 0, and a winner below
+// mag_tiny() is TMV's underflow (|a| < DBL_MIN / FLT_MIN), for which the
+// caller does not use the winner.
+__device__ __forceinline__ unsigned mag_hi(double a)
+{
+    const unsigned h = (unsigned)((unsigned long long)__double_as_longlong(a) >> 32) & 0x7fffffffu;
+    return a == a ? h : 0u;
+}
+__device__ __forceinline__ unsigned mag_hi(float a)
+{
+    const unsigned h = __float_as_uint(a) & 0x7fffffffu;
+    return a == a ? h : 0u;
+}
+__device__ __forceinline__ unsigned mag_lo(double a) { return (unsigned)__double_as_longlong(a); }
+__device__ __forceinline__ unsigned mag_lo(float) { return 0u; }
+template <typename T> __device__ __forceinline__ constexpr unsigned mag_tiny()
+{ return sizeof(T) == 8 ? 0x00100000u : 0x00800000u; }
+
+template <int CTRL, int RM>
+__device__ __forceinline__ unsigned dpp_umax_step(unsigned v)
+{
+    const unsigned o = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, RM, 0xf, false);
+    return v > o ? v : o;
+}
+
+template <int NL>
+__device__ __forceinline__ unsigned lanes_umax(unsigned v)
+{
+    static_assert(NL == 64 || NL == 16 || NL == 8 || NL == 4, "lanes 0..NL-1");
+    v = dpp_umax_step<0xB1, 0xf>(v);                             // quad_perm [1,0,3,2]
+    v = dpp_umax_step<0x4E, 0xf>(v);                             // quad_perm [2,3,0,1]
+    if constexpr (NL >= 8) v = dpp_umax_step<0x141, 0xf>(v);     // row_half_mirror
+    if constexpr (NL >= 16) v = dpp_umax_step<0x140, 0xf>(v);    // row_mirror
+    if constexpr (NL == 64) {
+        v = dpp_umax_step<0x142, 0xa>(v);                        // row_bcast:15
+        v = dpp_umax_step<0x143, 0xc>(v);                        // row_bcast:31
+    }
+    return (unsigned)__builtin_amdgcn_readlane((int)v, NL == 64 ? 63 : 0);
+}
+
+// The lane (of 0..NL-1) with the largest magnitude, lowest position on
+// ties; m receives its high key.  Positions of distinct candidates differ.
+template <int NL, typename T>
+__device__ __forceinline__ int lanes_best(unsigned hi, unsigned lo, int pos, unsigned& m)
+{
+    m = lanes_umax<NL>(hi);
+    constexpr unsigned long long in = NL == 64 ? ~0ull : (1ull << NL) - 1;
+    unsigned long long hit = __builtin_amdgcn_ballot_w64(hi == m) & in;
+    if ((hit & (hit - 1)) != 0ull && m >= mag_tiny<T>()) {
+        const int lane = threadIdx.x & 63;
+        if constexpr (sizeof(T) == 8) {
+            const unsigned l = lanes_umax<NL>(((hit >> lane) & 1) ? lo : 0u);
+            hit &= __builtin_amdgcn_ballot_w64(lo == l);
+        }
+        if ((hit & (hit - 1)) != 0ull) {
+            // lowest position = largest complement
+            const unsigned q = lanes_umax<NL>(((hit >> lane) & 1) ? ~(unsigned)pos : 0u);
+            hit &= __builtin_amdgcn_ballot_w64(~(unsigned)pos == q);
+        }
+    }
+    return (int)__builtin_ctzll(hit);
 }
 
 } // namespace tmvx

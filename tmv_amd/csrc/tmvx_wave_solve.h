@@ -1,6 +1,7 @@
 // One-wave solves with stored LU factors (n <= WS_NMAX), lane-distributed
 // vectors: lane l holds entries l + 64 s, s < WS_PR.  Shared by the batched
-// solve and the adjoint kernels.
+// solve and the adjoint kernels, for batches large enough to fill the GPU
+// with one wave per system (smaller ones: tmvx_wg_solve.h).
 //
 // A x = b: permute by the interchange list, then unit-lower L and U by
 // column sweeps (TMV LU_LDivEq, src/TMV_LUDiv.cpp:185-226, with the

@@ -1,0 +1,256 @@
+// Solves with stored LU factors of one small system (n <= WS_NMAX), by one
+// workgroup or one wave, up to 16 right-hand sides at a time, for batches
+// that leave the GPU short of waves.  Shared by the batched solve and the
+// adjoint.
+//
+// A X = B: rows gathered through the interchange list, then unit-lower L and
+// U (TMV LU_LDivEq, src/TMV_LUDiv.cpp:185-226).  A^T X = B: U^T, then L^T,
+// then the rows scattered back (TMV LU_RDivEq on B^T, src/TMV_LUDiv.cpp:
+// 369-410).  Entries are divided by U's diagonal, a zero entry stays zero
+// (src/TMV_TriDiv_V.cpp:187).
+//
+// The triangle is walked in blocks of 16 rows.  The right-hand sides still
+// to be solved are MFMA accumulators (16 rows x 16 right-hand sides each,
+// the 16-row blocks dealt out to the waves); a solved block's product with
+// the rows to come is one 16x16x16 MFMA step per block row, with the factor
+// entries loaded a block ahead.  The diagonal block itself is a plain
+// substitution, a right-hand side per lane, its entries broadcast from LDS.
+// One barrier per block: the chain is 16 substitution steps per block
+// instead of a wave-wide sweep (or a wave sum, for A^T) per row, and four
+// waves stream the factors of one system.
+#pragma once
+#include "tmvx_wave_solve.h"
+
+namespace tmvx {
+
+// Batches of up to this many systems take the workgroup form; larger ones
+// fill the GPU with a wave per system (tmvx_wave_solve.h), which keeps
+// eight systems in flight where this form, by its LDS, keeps two: measured
+// FP64 with one right-hand side, 512 systems of n = 256 314 -> 143 us
+// (transposed 286 -> 136), n = 200 135 -> 94 us, 300 of n = 64 42 -> 28 us,
+// but 2000 of n = 128 97 -> 224 us and 4000 of n = 65 91 -> 234 us.
+constexpr int WS_WG_MAX = 1024;
+
+constexpr int WS_RHS = 16;                 // right-hand sides per pass
+constexpr int WS_TPW = 4;                  // 16-row blocks per wave
+
+struct GroupSync {
+    __device__ __forceinline__ void operator()() const { __syncthreads(); }
+};
+struct WaveSync {
+    __device__ __forceinline__ void operator()() const
+    {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    }
+};
+
+// LDS of one system solved by NWV waves (n <= 64 NWV).
+template <typename T, int NWV>
+struct WgSolveLds {
+    static constexpr int NMAX = 16 * WS_TPW * NWV;
+    T x[NMAX][WS_RHS];
+    T d[NMAX / 16][16][16];                // d[b][k][i] = op(A)(16 b + i, 16 b + k)
+    short src[NMAX];                       // row i of P A is row src[i] of A
+    short piv[NMAX];
+};
+
+// One triangular solve on L.x (rows past n are zero).  LOWER: op(A) is
+// lower triangular (walked forward).
+template <typename T, int NWV, bool TRANS, bool LOWER, bool UNIT, class Sync>
+__device__ __forceinline__ void wg_trsv(int n, const T* __restrict__ A, WgSolveLds<T, NWV>& L,
+                                        int tid, Sync sync)
+{
+    typedef typename Mfma<T>::v4 v4;
+    const int lane = tid & 63, wave = NWV == 1 ? 0 : tid >> 6, li = lane & 15, g = lane >> 4;
+    const int nb = (n + 15) >> 4;
+    const i64 ld = n;
+    for (int e = tid; e < nb * 256; e += 64 * NWV) {
+        const int b = e >> 8, i = 16 * b + (TRANS ? (e >> 4) & 15 : e & 15);
+        const int k = 16 * b + (TRANS ? e & 15 : (e >> 4) & 15);
+        L.d[b][k & 15][i & 15] = (i < n && k < n) ? (TRANS ? A[k + i * ld] : A[i + k * ld])
+                                                  : (i == k ? T(1) : T(0));
+    }
+    // op(A)(16 tb + li, 16 b + k(s, g)), the MFMA k slot (s, g) holding
+    // k = 4 s + g, or 4 g + s where k is the contiguous index of A
+    auto frag = [&](int tb, int b, T (&f)[4]) __attribute__((always_inline)) {
+        const int r = 16 * tb + li, rc = r < n ? r : n - 1;
+        static_for<0, 4>([&](auto sc) __attribute__((always_inline)) {
+            constexpr int s = decltype(sc)::value;
+            const int k = 16 * b + (TRANS ? 4 * g + s : 4 * s + g), kc = k < n ? k : n - 1;
+            const T v = TRANS ? A[kc + rc * ld] : A[rc + kc * ld];
+            f[s] = (r < n && k < n) ? v : T(0);
+        });
+    };
+    auto later = [&](int tb, int b) __attribute__((always_inline)) {
+        return LOWER ? (tb > b && tb < nb) : tb < b;
+    };
+    v4 acc[WS_TPW];
+    T f[WS_TPW][4];
+    const int first = LOWER ? 0 : nb - 1;
+    static_for<0, WS_TPW>([&](auto tc) __attribute__((always_inline)) {
+        constexpr int t = decltype(tc)::value;
+        const int tb = wave + NWV * t;
+        static_for<0, 4>([&](auto rc) __attribute__((always_inline)) {
+            constexpr int r = decltype(rc)::value;
+            acc[t][r] = L.x[16 * tb + Mfma<T>::row(g, r)][li];
+        });
+        if (later(tb, first)) frag(tb, first, f[t]);
+    });
+    sync();                                   // L.d complete
+    for (int q = 0; q < nb; ++q) {
+        const int b = LOWER ? q : nb - 1 - q, bn = LOWER ? b + 1 : b - 1;
+        if (NWV == 1 || wave == b % NWV) {
+            // the block's right-hand sides through LDS to one per lane
+            // (every lane group solves the same 16)
+            T x[16];
+            static_for<0, 16>([&](auto kc) __attribute__((always_inline)) {
+                constexpr int k = decltype(kc)::value;
+                x[k] = L.x[16 * b + k][li];
+            });
+            // column k of the diagonal block is read one step before its use
+            // (the offset passes through an empty asm statement with the
+            // previous entry, or all 120 reads would be hoisted to the top)
+            T d[16];
+            int off = 0;
+            auto dcol = [&](auto kc, T (&c)[16]) __attribute__((always_inline)) {
+                constexpr int k = decltype(kc)::value;
+                static_for<0, 16>([&](auto ic) __attribute__((always_inline)) {
+                    constexpr int i = decltype(ic)::value;
+                    if constexpr ((LOWER ? i > k : i < k) || (!UNIT && i == k)) c[i] = (&L.d[b][k][i])[off];
+                });
+            };
+            dcol(std::integral_constant<int, LOWER ? 0 : 15>{}, d);
+            static_for<0, 16>([&](auto qc) __attribute__((always_inline)) {
+                constexpr int q = decltype(qc)::value, k = LOWER ? q : 15 - q;
+                T dn[16];
+                if constexpr (q > 0) __asm__ volatile("" : "+v"(off) : "v"(x[k]));
+                if constexpr (q < 15) dcol(std::integral_constant<int, LOWER ? k + 1 : k - 1>{}, dn);
+                if constexpr (!UNIT) x[k] = x[k] == T(0) ? T(0) : x[k] / d[k];
+                static_for<0, 16>([&](auto ic) __attribute__((always_inline)) {
+                    constexpr int i = decltype(ic)::value;
+                    if constexpr (LOWER ? i > k : i < k) x[i] -= d[i] * x[k];
+                    if constexpr (q < 15) d[i] = dn[i];
+                });
+            });
+            if (g == 0)
+                static_for<0, 16>([&](auto kc) __attribute__((always_inline)) {
+                    constexpr int k = decltype(kc)::value;
+                    L.x[16 * b + k][li] = x[k];
+                });
+        }
+        sync();
+        if (bn < 0 || bn >= nb) break;
+        // the next block first: its owner goes on with it
+        T xb[4];
+        static_for<0, 4>([&](auto sc) __attribute__((always_inline)) {
+            constexpr int s = decltype(sc)::value;
+            xb[s] = L.x[16 * b + (TRANS ? 4 * g + s : 4 * s + g)][li];
+        });
+        static_for<0, 2>([&](auto pc) __attribute__((always_inline)) {
+            static_for<0, WS_TPW>([&](auto tc) __attribute__((always_inline)) {
+                constexpr int t = decltype(tc)::value;
+                const int tb = wave + NWV * t;
+                if ((tb == bn) != (decltype(pc)::value == 0) || !later(tb, b)) return;   // uniform
+                static_for<0, 4>([&](auto sc) __attribute__((always_inline)) {
+                    constexpr int s = decltype(sc)::value;
+                    acc[t] = Mfma<T>::mac(-f[t][s], xb[s], acc[t]);
+                });
+                if constexpr (decltype(pc)::value == 0)
+                    static_for<0, 4>([&](auto rc) __attribute__((always_inline)) {
+                        constexpr int r = decltype(rc)::value;
+                        L.x[16 * tb + Mfma<T>::row(g, r)][li] = acc[t][r];
+                    });
+            });
+        });
+        static_for<0, WS_TPW>([&](auto tc) __attribute__((always_inline)) {
+            constexpr int t = decltype(tc)::value;
+            const int tb = wave + NWV * t;
+            if (later(tb, bn)) frag(tb, bn, f[t]);       // in flight during the next block
+        });
+        WaveSync()();                         // the owner's block is in LDS for its own reads
+    }
+}
+
+// X := A^-1 B (A^-T B) for nr right-hand sides, B and X n x nr with leading
+// dimension n (X may be B).
+template <typename T, int NWV, bool TRANS, class Sync>
+__device__ __forceinline__ void wg_getrs(int n, int nr, const T* __restrict__ LU,
+                                         const i64* __restrict__ piv, const T* B, T* X,
+                                         WgSolveLds<T, NWV>& L, int tid, Sync sync)
+{
+    constexpr int NT = 64 * NWV;
+    for (int i = tid; i < n; i += NT) {
+        const i64 p = piv[i];
+        L.piv[i] = (short)((p >= 0 && p < n) ? p : i);
+    }
+    sync();
+    // the row that the interchanges, taken backwards, trace row i to
+    for (int i = tid; i < n; i += NT) {
+        int s = i;
+        for (int k = n - 1; k >= 0; --k) {
+            const int p = L.piv[k];
+            s = s == k ? p : s == p ? k : s;
+        }
+        L.src[i] = (short)s;
+    }
+    sync();
+    const int nb = (n + 15) >> 4;
+    for (int c0 = 0; c0 < nr; c0 += WS_RHS) {
+        const int nc = nr - c0 < WS_RHS ? nr - c0 : WS_RHS;
+        for (int e = tid; e < nb * 256; e += NT) {
+            const int i = e % (nb * 16), c = e / (nb * 16);
+            T v = T(0);
+            if (i < n && c < nc) v = B[(TRANS ? i : (int)L.src[i]) + (i64)(c0 + c) * n];
+            L.x[i][c] = v;
+        }
+        sync();
+        if constexpr (!TRANS) {
+            wg_trsv<T, NWV, false, true, true>(n, LU, L, tid, sync);
+            wg_trsv<T, NWV, false, false, false>(n, LU, L, tid, sync);
+        } else {
+            wg_trsv<T, NWV, true, true, false>(n, LU, L, tid, sync);
+            wg_trsv<T, NWV, true, false, true>(n, LU, L, tid, sync);
+        }
+        for (int e = tid; e < nc * n; e += NT) {
+            const int i = e % n, c = e / n;
+            X[(TRANS ? (int)L.src[i] : i) + (i64)(c0 + c) * n] = L.x[i][c];
+        }
+        sync();
+    }
+}
+
+// The systems of a batch: a workgroup of four waves takes one system with
+// 64 < n <= WS_NMAX at a time, a wave one with n <= 64 (larger ones are
+// skipped).
+template <typename T>
+union WgSolveShared {
+    WgSolveLds<T, 4> g;
+    WgSolveLds<T, 1> w[4];
+};
+
+template <typename T, bool TRANS>
+__device__ __forceinline__ void wg_getrs_batch(int count, const int* __restrict__ nv,
+                                               const int* __restrict__ nrhsv,
+                                               const T* const* __restrict__ LUv,
+                                               const i64* const* __restrict__ pivv,
+                                               const T* const* Bv, T* const* Xv,
+                                               WgSolveShared<T>& sh)
+{
+    const int tid = threadIdx.x, wave = tid >> 6;
+    for (int sys = blockIdx.x; sys < count; sys += gridDim.x) {
+        const int n = nv[sys], nr = nrhsv[sys];
+        if (n <= 64 || n > WS_NMAX || nr <= 0) continue;
+        wg_getrs<T, 4, TRANS>(n, nr, LUv[sys], pivv[sys], Bv[sys], Xv[sys], sh.g, tid, GroupSync());
+    }
+    __syncthreads();
+    for (int sys = (int)blockIdx.x * 4 + wave; sys < count; sys += (int)gridDim.x * 4) {
+        const int n = nv[sys], nr = nrhsv[sys];
+        if (n <= 0 || n > 64 || nr <= 0) continue;
+        wg_getrs<T, 1, TRANS>(n, nr, LUv[sys], pivv[sys], Bv[sys], Xv[sys], sh.w[wave], tid & 63,
+                              WaveSync());
+    }
+}
+
+} // namespace tmvx
