@@ -5,7 +5,7 @@
  * system with LU_Decompose + LU_LDivEq (src/TMV_LUDecompose.cpp:514-559,
  * src/TMV_LUDiv.cpp:185-226) or x = b/m with divideUsing(LU), and
  * multiplies with MultMM (src/TMV_MultMM.cpp:404-477), in a loop.  These
- * entry points do the whole loop in one launch with the same per-system
+ * entry points do the whole loop in a few launches with the same per-system
  * semantics: pivots are TMV's interchange list (0-based, first maximum in
  * the current row order, TMV's underflow rule), factors in place.
  *
@@ -30,11 +30,9 @@ typedef struct tmvx_batch_plan_s* tmvx_batch_plan;
 /*
  * A plan for a batch of `count` systems of orders n_host[i] (1..128) with
  * nrhs_host[i] (0..16; NULL = 0: factor only) right-hand sides, in FP64 or
- * FP32.  The plan orders the work list (largest systems first) and picks
- * the launch schedule: which systems run one per wave and which one per
- * 256-thread workgroup, and how many workgroups per CU.  tune != 0 times
- * every candidate schedule on a synthetic batch of the same sizes and
- * keeps the fastest; tune == 0 keeps the default (waves for n <= 32).
+ * FP32.  The plan orders the work list (largest systems first): systems of
+ * n <= 64 run one per wave, larger ones one per 128-thread workgroup.
+ * tune != 0 also times the plan on a synthetic batch of the same sizes.
  * Allocates device memory and synchronises `stream`; not capturable.
  */
 int tmvx_batch_plan_create(int dtype, int64_t count, const int32_t* n_host,
@@ -44,7 +42,8 @@ int tmvx_batch_plan_destroy(tmvx_batch_plan plan);
 /* Text naming the plan's schedule (valid until the plan changes). */
 const char* tmvx_batch_plan_describe(tmvx_batch_plan plan);
 /* Force a schedule: index < tmvx_batch_schedule_count(), wave split,
- * workgroups per CU.  For tuning experiments and tests. */
+ * workgroups per CU (1..16).  For tuning experiments and tests: every choice
+ * gives the same results. */
 int tmvx_batch_plan_set(tmvx_batch_plan plan, int schedule, int split, int wgs_per_cu,
                         void* stream);
 int tmvx_batch_schedule_count(void);
@@ -55,8 +54,8 @@ int tmvx_batch_schedule_count(void);
  * interchanges; info[i] (device) the 1-based index of the first zero pivot
  * or 0.  For a system with info[i] > 0 the factorisation is complete (TMV's
  * zero-column rule) but B[i] is left unspecified, as LAPACK gesv leaves it.
- * One kernel launch on `stream`: no allocation, no host synchronisation,
- * no memset -- safe to capture in a hipGraph and replay.
+ * Up to three kernel launches on `stream`: no allocation, no host
+ * synchronisation, no memset -- safe to capture in a hipGraph and replay.
  * Per system: TMV LU_Decompose (src/TMV_LUDecompose.cpp:514-559) followed
  * by LU_LDivEq (src/TMV_LUDiv.cpp:185-226).
  */

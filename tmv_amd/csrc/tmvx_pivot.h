@@ -169,13 +169,13 @@ __device__ __forceinline__ int lanes_best(unsigned hi, unsigned lo, int pos, uns
     m = lanes_umax<NL>(hi);
     constexpr unsigned long long in = NL == 64 ? ~0ull : (1ull << NL) - 1;
     unsigned long long hit = __builtin_amdgcn_ballot_w64(hi == m) & in;
-    if ((hit & (hit - 1)) != 0ull && m >= mag_tiny<T>()) {
+    if (__builtin_popcountll(hit) > 1 && m >= mag_tiny<T>()) {
         const int lane = threadIdx.x & 63;
         if constexpr (sizeof(T) == 8) {
             const unsigned l = lanes_umax<NL>(((hit >> lane) & 1) ? lo : 0u);
             hit &= __builtin_amdgcn_ballot_w64(lo == l);
         }
-        if ((hit & (hit - 1)) != 0ull) {
+        if (__builtin_popcountll(hit) > 1) {
             // lowest position = largest complement
             const unsigned q = lanes_umax<NL>(((hit >> lane) & 1) ? ~(unsigned)pos : 0u);
             hit &= __builtin_amdgcn_ballot_w64(~(unsigned)pos == q);
@@ -183,5 +183,59 @@ __device__ __forceinline__ int lanes_best(unsigned hi, unsigned lo, int pos, uns
     }
     return (int)__builtin_ctzll(hit);
 }
+
+// Lane C of each row of 16 lanes, in all 16 (DPP row_newbcast): one move
+// where a v_readlane of the same value makes the next vector instruction
+// wait for its scalar register (~37 cycles each in a chain of them).  Call
+// with every lane active.
+template <int C>
+__device__ __forceinline__ double row_bcast(double v)
+{
+    static_assert(C >= 0 && C < 16, "lane of a row");
+    return __longlong_as_double(__builtin_amdgcn_update_dpp(
+        0l, (long)__double_as_longlong(v), 0x150 + C, 0xf, 0xf, true));
+}
+template <int C>
+__device__ __forceinline__ float row_bcast(float v)
+{
+    static_assert(C >= 0 && C < 16, "lane of a row");
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + C, 0xf, 0xf,
+                                                      true));
+}
+
+// r[c] += (lane 8 H + c of each row of 16 lanes of u) * l, c < 8: broadcast
+// and multiply-add in one instruction (v_fmac with DPP row_newbcast, which the
+// compiler does not form by itself; as moves and multiply-adds apart, they
+// also get apart, and the moves' results spill).  Call with every lane active.
+// The leading s_nop: a DPP operand is not read within two wait states of the
+// vector instruction that wrote it.
+#define TMVX_FMAC8(SUF, A, B, C, D, E, F, G, I)                                                 \
+    __asm__ volatile("s_nop 1\n\t"                                                              \
+                     "v_fmac_" SUF "_dpp %0, %8, %9 row_newbcast:" A " row_mask:0xf bank_mask:0xf\n\t" \
+                     "v_fmac_" SUF "_dpp %1, %8, %9 row_newbcast:" B " row_mask:0xf bank_mask:0xf\n\t" \
+                     "v_fmac_" SUF "_dpp %2, %8, %9 row_newbcast:" C " row_mask:0xf bank_mask:0xf\n\t" \
+                     "v_fmac_" SUF "_dpp %3, %8, %9 row_newbcast:" D " row_mask:0xf bank_mask:0xf\n\t" \
+                     "v_fmac_" SUF "_dpp %4, %8, %9 row_newbcast:" E " row_mask:0xf bank_mask:0xf\n\t" \
+                     "v_fmac_" SUF "_dpp %5, %8, %9 row_newbcast:" F " row_mask:0xf bank_mask:0xf\n\t" \
+                     "v_fmac_" SUF "_dpp %6, %8, %9 row_newbcast:" G " row_mask:0xf bank_mask:0xf\n\t" \
+                     "v_fmac_" SUF "_dpp %7, %8, %9 row_newbcast:" I " row_mask:0xf bank_mask:0xf"   \
+                     : "+v"(r[C0]), "+v"(r[C0 + 1]), "+v"(r[C0 + 2]), "+v"(r[C0 + 3]),              \
+                       "+v"(r[C0 + 4]), "+v"(r[C0 + 5]), "+v"(r[C0 + 6]), "+v"(r[C0 + 7])          \
+                     : "v"(u), "v"(l))
+template <int H, int C0, int N, typename T>
+__device__ __forceinline__ void bcast_fma8(T (&r)[N], T u, T l)
+{
+    static_assert((H == 0 || H == 1) && C0 >= 0 && C0 + 8 <= N, "eight entries");
+#ifdef __HIP_DEVICE_COMPILE__
+    if constexpr (sizeof(T) == 8) {
+        if constexpr (H == 0) TMVX_FMAC8("f64", "0", "1", "2", "3", "4", "5", "6", "7");
+        else TMVX_FMAC8("f64", "8", "9", "10", "11", "12", "13", "14", "15");
+    } else {
+        if constexpr (H == 0) TMVX_FMAC8("f32", "0", "1", "2", "3", "4", "5", "6", "7");
+        else TMVX_FMAC8("f32", "8", "9", "10", "11", "12", "13", "14", "15");
+    }
+#endif
+}
+#undef TMVX_FMAC8
 
 } // namespace tmvx

@@ -37,12 +37,14 @@ constexpr int WS_TPW = 4;                  // 16-row blocks per wave
 struct GroupSync {
     __device__ __forceinline__ void operator()() const { __syncthreads(); }
 };
+// Between the lanes of one wave: its LDS and memory accesses are in order, so
+// only the compiler is held back.
 struct WaveSync {
     __device__ __forceinline__ void operator()() const
     {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
 };
 
@@ -56,16 +58,15 @@ struct WgSolveLds {
     short piv[NMAX];
 };
 
-// One triangular solve on L.x (rows past n are zero).  LOWER: op(A) is
-// lower triangular (walked forward).
+// One triangular solve on L.x (rows past n are zero), A with leading
+// dimension ld.  LOWER: op(A) is lower triangular (walked forward).
 template <typename T, int NWV, bool TRANS, bool LOWER, bool UNIT, class Sync>
-__device__ __forceinline__ void wg_trsv(int n, const T* __restrict__ A, WgSolveLds<T, NWV>& L,
-                                        int tid, Sync sync)
+__device__ __forceinline__ void wg_trsv(int n, const T* __restrict__ A, int ld,
+                                        WgSolveLds<T, NWV>& L, int tid, Sync sync)
 {
     typedef typename Mfma<T>::v4 v4;
     const int lane = tid & 63, wave = NWV == 1 ? 0 : tid >> 6, li = lane & 15, g = lane >> 4;
     const int nb = (n + 15) >> 4;
-    const i64 ld = n;
     for (int e = tid; e < nb * 256; e += 64 * NWV) {
         const int b = e >> 8, i = 16 * b + (TRANS ? (e >> 4) & 15 : e & 15);
         const int k = 16 * b + (TRANS ? e & 15 : (e >> 4) & 15);
@@ -200,18 +201,18 @@ __device__ __forceinline__ void wg_getrs(int n, int nr, const T* __restrict__ LU
     for (int c0 = 0; c0 < nr; c0 += WS_RHS) {
         const int nc = nr - c0 < WS_RHS ? nr - c0 : WS_RHS;
         for (int e = tid; e < nb * 256; e += NT) {
-            const int i = e % (nb * 16), c = e / (nb * 16);
+            const int i = e % (nb * 16), c = e / (nb * 16);    // (c < 16)
             T v = T(0);
             if (i < n && c < nc) v = B[(TRANS ? i : (int)L.src[i]) + (i64)(c0 + c) * n];
             L.x[i][c] = v;
         }
         sync();
         if constexpr (!TRANS) {
-            wg_trsv<T, NWV, false, true, true>(n, LU, L, tid, sync);
-            wg_trsv<T, NWV, false, false, false>(n, LU, L, tid, sync);
+            wg_trsv<T, NWV, false, true, true>(n, LU, n, L, tid, sync);
+            wg_trsv<T, NWV, false, false, false>(n, LU, n, L, tid, sync);
         } else {
-            wg_trsv<T, NWV, true, true, false>(n, LU, L, tid, sync);
-            wg_trsv<T, NWV, true, false, true>(n, LU, L, tid, sync);
+            wg_trsv<T, NWV, true, true, false>(n, LU, n, L, tid, sync);
+            wg_trsv<T, NWV, true, false, true>(n, LU, n, L, tid, sync);
         }
         for (int e = tid; e < nc * n; e += NT) {
             const int i = e % n, c = e / n;
@@ -221,9 +222,10 @@ __device__ __forceinline__ void wg_getrs(int n, int nr, const T* __restrict__ LU
     }
 }
 
-// The systems of a batch: a workgroup of four waves takes one system with
-// 64 < n <= WS_NMAX at a time, a wave one with n <= 64 (larger ones are
-// skipped).
+// The systems of a batch, with a grid of one workgroup per system: workgroup
+// i takes system i when 64 < n <= WS_NMAX, wave i of the grid system i when
+// n <= 64 (larger ones are skipped).  No loop over systems: what a loop could
+// keep in registers from one to the next is more than there are.
 template <typename T>
 union WgSolveShared {
     WgSolveLds<T, 4> g;
@@ -238,19 +240,24 @@ __device__ __forceinline__ void wg_getrs_batch(int count, const int* __restrict_
                                                const T* const* Bv, T* const* Xv,
                                                WgSolveShared<T>& sh)
 {
-    const int tid = threadIdx.x, wave = tid >> 6;
-    for (int sys = blockIdx.x; sys < count; sys += gridDim.x) {
-        const int n = nv[sys], nr = nrhsv[sys];
-        if (n <= 64 || n > WS_NMAX || nr <= 0) continue;
-        wg_getrs<T, 4, TRANS>(n, nr, LUv[sys], pivv[sys], Bv[sys], Xv[sys], sh.g, tid, GroupSync());
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    {
+        const int sys = blockIdx.x;
+        const int n = __builtin_amdgcn_readfirstlane(nv[sys]);
+        const int nr = __builtin_amdgcn_readfirstlane(nrhsv[sys]);
+        if (n > 64 && n <= WS_NMAX && nr > 0)
+            wg_getrs<T, 4, TRANS>(n, nr, LUv[sys], pivv[sys], Bv[sys], Xv[sys], sh.g, tid,
+                                  GroupSync());
     }
+    if ((int)blockIdx.x * 4 >= count) return;
     __syncthreads();
-    for (int sys = (int)blockIdx.x * 4 + wave; sys < count; sys += (int)gridDim.x * 4) {
-        const int n = nv[sys], nr = nrhsv[sys];
-        if (n <= 0 || n > 64 || nr <= 0) continue;
+    const int sys = (int)blockIdx.x * 4 + wave;
+    if (sys >= count) return;
+    const int n = __builtin_amdgcn_readfirstlane(nv[sys]);
+    const int nr = __builtin_amdgcn_readfirstlane(nrhsv[sys]);
+    if (n > 0 && n <= 64 && nr > 0)
         wg_getrs<T, 1, TRANS>(n, nr, LUv[sys], pivv[sys], Bv[sys], Xv[sys], sh.w[wave], tid & 63,
                               WaveSync());
-    }
 }
 
 } // namespace tmvx
