@@ -9,17 +9,32 @@
 // itself (src/TMV_LUDecompose.cpp:162-169); the column below the pivot is
 // scaled by the pivot's reciprocal.
 //
-// Blocked right-looking, 64-column panels:
-//   panel: ONE workgroup factors the panel column by column (pivot search
-//     by a block reduction, the interchange applied to the whole row, the
-//     column scaled and the panel's remaining columns updated); a simple,
-//     latency-bound form -- the complex path is not a measured workload;
-//   U12 = L11^-1 A12: one thread per column;
-//   A22 -= L21 U12: the complex GEMM (four real MFMA products).
-// Solves: interchanges by one thread per right-hand side, then triangular
-// column sweeps by one workgroup per right-hand side.
-#include "tmvx_common.h"
+// While more than ZN_MMAX rows are left: 64-column panels, each by ONE
+// workgroup column by column in global memory, U12 by one thread per column,
+// A22 -= L21 U12 on the complex GEMM.
+// From there on (the whole of a system up to that order): panels of 16 (8)
+// columns, two launches each:
+//   znpanel_kernel: one workgroup, its rows in registers (one to four a
+//     thread).  Rows never move: each carries its position.  Per column one
+//     barrier: every wave's best row (largest modulus, found on integer keys)
+//     goes to LDS with the reciprocal of its pivot, every wave picks the
+//     winner and updates its rows, the pivot row's entries handed on by DPP
+//     broadcasts;
+//   znupdate_kernel: 8 columns per workgroup: U12 with a row per lane, then the
+//     rank-16 update with a row of L21 per lane; the interchanges are the rows
+//     that the update reads from.
+// The interchanges of the columns to the left are applied once, at the end.
+// Solves up to ZS_NMAX: one workgroup per right-hand side, the vector in LDS,
+// 16 rows at a time (substitution on 16 lanes, then the rows to come with the
+// next 16 columns already loaded); above: column sweeps by one workgroup.
+// Bound: the panel's chain (1.3-1.8 us a column, most of it hypot, the pivot's
+// reciprocal and one barrier) and two launches per 16 columns.  Measured at
+// n = 1000, 4 right-hand sides, FP64: 22.1 -> 3.1 ms (panels 12.0 -> 1.6, U12
+// and update 5.8 -> 0.7, solves 2.9 -> 0.6, left interchanges 0.1).
+#include "tmvx_lu.h"
+#include "tmvx_pivot.h"
 
+#include <algorithm>
 #include <cfloat>
 
 namespace tmvx {
@@ -163,6 +178,328 @@ __global__ void ztrsm_u12_kernel(i64 n, typename CplxT<R>::type* __restrict__ A,
     }
 }
 
+// ---- panels in registers -------------------------------------------------
+
+constexpr int ZN_NTH = 512;              // panel workgroup
+constexpr int ZN_NW = ZN_NTH / 64;
+constexpr i64 ZN_MMAX = 4 * ZN_NTH;      // rows a panel can hold (four a thread)
+
+// x -= l u
+template <typename Z> __device__ __forceinline__ void csubmul(Z& x, Z l, Z u)
+{
+    x.x = fma(-l.x, u.x, fma(l.y, u.y, x.x));
+    x.y = fma(-l.x, u.y, fma(-l.y, u.x, x.y));
+}
+template <int C, typename Z> __device__ __forceinline__ Z row_bcast_z(Z v)
+{
+    Z r;
+    r.x = row_bcast<C>(v.x);
+    r.y = row_bcast<C>(v.y);
+    return r;
+}
+
+// x -= sum over k in [K0, K0 + 4) of l[k] (lane k of each row of 16 lanes of u),
+// given -u.x, -u.y and u.y: broadcast and multiply-add in one instruction
+// (cf. bcast_fma8).  Call with every lane active.
+#define ZN_STEP(SUF, K, LX, LY)                                                              \
+    "v_fmac_" SUF "_dpp %0, %2, " LX " row_newbcast:" K " row_mask:0xf bank_mask:0xf\n\t"      \
+    "v_fmac_" SUF "_dpp %1, %3, " LX " row_newbcast:" K " row_mask:0xf bank_mask:0xf\n\t"      \
+    "v_fmac_" SUF "_dpp %0, %4, " LY " row_newbcast:" K " row_mask:0xf bank_mask:0xf\n\t"      \
+    "v_fmac_" SUF "_dpp %1, %2, " LY " row_newbcast:" K " row_mask:0xf bank_mask:0xf\n\t"
+#define ZN_FMAC4(SUF, A, B, C, D)                                                            \
+    __asm__ volatile("s_nop 1\n\t" ZN_STEP(SUF, A, "%5", "%9") ZN_STEP(SUF, B, "%6", "%10")   \
+                         ZN_STEP(SUF, C, "%7", "%11") ZN_STEP(SUF, D, "%8", "%12")           \
+                     : "+v"(xr), "+v"(xi)                                                    \
+                     : "v"(nux), "v"(nuy), "v"(uy), "v"(l[K0].x), "v"(l[K0 + 1].x),          \
+                       "v"(l[K0 + 2].x), "v"(l[K0 + 3].x), "v"(l[K0].y), "v"(l[K0 + 1].y),   \
+                       "v"(l[K0 + 2].y), "v"(l[K0 + 3].y))
+template <int K0, typename R, typename Z, int N>
+__device__ __forceinline__ void zbcast_fma4(R& xr, R& xi, R nux, R nuy, R uy, const Z (&l)[N])
+{
+    static_assert(K0 % 4 == 0 && K0 < 16 && K0 + 4 <= N, "four of sixteen lanes");
+#ifdef __HIP_DEVICE_COMPILE__
+    if constexpr (sizeof(R) == 8) {
+        if constexpr (K0 == 0) ZN_FMAC4("f64", "0", "1", "2", "3");
+        else if constexpr (K0 == 4) ZN_FMAC4("f64", "4", "5", "6", "7");
+        else if constexpr (K0 == 8) ZN_FMAC4("f64", "8", "9", "10", "11");
+        else ZN_FMAC4("f64", "12", "13", "14", "15");
+    } else {
+        if constexpr (K0 == 0) ZN_FMAC4("f32", "0", "1", "2", "3");
+        else if constexpr (K0 == 4) ZN_FMAC4("f32", "4", "5", "6", "7");
+        else if constexpr (K0 == 8) ZN_FMAC4("f32", "8", "9", "10", "11");
+        else ZN_FMAC4("f32", "12", "13", "14", "15");
+    }
+#endif
+}
+#undef ZN_FMAC4
+#undef ZN_STEP
+
+// Columns [j0, j0 + jb) of the m = n - j0 rows from j0 on, m <= RPT ZN_NTH:
+// row t + q ZN_NTH of the panel in thread t's slot q.  from[r]: the panel-
+// relative row that ends at position r.
+template <typename R, int RPT, int NB>
+__global__ void __launch_bounds__(ZN_NTH)
+znpanel_kernel(i64 n, typename CplxT<R>::type* __restrict__ Ag, i64 lda, i64 j0, int jb,
+               i64* __restrict__ piv, i64* __restrict__ first_zero, int* __restrict__ from)
+{
+    typedef typename CplxT<R>::type Z;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int m = (int)(n - j0);
+    Z* __restrict__ A = Ag + j0 + j0 * lda;
+    __shared__ __attribute__((aligned(16))) Z s_row[2][ZN_NW][16];
+    __shared__ unsigned s_hi[2][ZN_NW], s_lo[2][ZN_NW];
+    __shared__ int s_pos[2][ZN_NW];
+    Z row[RPT][NB];
+    int pos[RPT];
+    bool used[RPT];
+    static_for<0, RPT>([&](auto q_) __attribute__((always_inline)) {
+        constexpr int q = decltype(q_)::value;
+        const int r = t + q * ZN_NTH;
+        pos[q] = r;
+        used[q] = r >= m;
+#pragma unroll
+        for (int c = 0; c < NB; ++c) {
+            Z z;
+            z.x = z.y = R(0);
+            if (r < m && c < jb) z = A[r + c * lda];
+            row[q][c] = z;
+        }
+    });
+    // (columns past jb run as zero columns, with nothing recorded)
+    static_for<0, NB>([&](auto kc) __attribute__((always_inline)) {
+        constexpr int k = decltype(kc)::value, par = k & 1;
+        // the thread's best row: largest modulus, lowest position
+        unsigned hi = 0u, lo = 0u;
+        int bp = INT_MAX, bq = 0;
+        static_for<0, RPT>([&](auto q_) __attribute__((always_inline)) {
+            constexpr int q = decltype(q_)::value;
+            const R v = R(hypot(row[q][k].x, row[q][k].y));
+            const unsigned h = mag_hi(v), l = mag_lo(v);
+            if (!used[q] && (bp == INT_MAX || h > hi || (h == hi && (l > lo || (l == lo && pos[q] < bp))))) {
+                hi = h; lo = l; bp = pos[q]; bq = q;
+            }
+        });
+        unsigned gm;
+        const int wl = lanes_best<64, R>(hi, lo, bp, gm);
+        if (lane == wl) {
+            s_hi[par][wave] = hi;
+            s_lo[par][wave] = lo;
+            s_pos[par][wave] = bp;
+        }
+        const int bu = __builtin_amdgcn_readlane(bq, wl);
+        static_for<0, RPT>([&](auto q_) __attribute__((always_inline)) {
+            constexpr int q = decltype(q_)::value;
+            if (bu == q) {                             // uniform
+                Z one;
+                one.x = R(1);
+                one.y = R(0);
+                const Z inv = cdiv(one, row[q][k]);    // in place of the pivot
+                if (lane == wl) {
+                    s_row[par][wave][k] = inv;
+                    static_for<k + 1, NB>([&](auto cc) __attribute__((always_inline)) {
+                        constexpr int c = decltype(cc)::value;
+                        s_row[par][wave][c] = row[q][c];
+                    });
+                }
+                __asm__ volatile("" ::: "memory");     // (keeps the slots' code apart: merged,
+                                                       // it would index the rows in memory)
+            }
+        });
+        __syncthreads();
+        const int cp = s_pos[par][lane & (ZN_NW - 1)];
+        const int ww = lanes_best<8, R>(s_hi[par][lane & (ZN_NW - 1)], s_lo[par][lane & (ZN_NW - 1)],
+                                        cp, gm);
+        const bool zero = gm < mag_tiny<R>();                         // TMV_Underflow
+        const int p = zero ? k : __builtin_amdgcn_readlane(cp, ww);
+        const Z uv = s_row[par][ww][lane & 15];        // lane li: entry li of the pivot row
+        if (t == 0 && k < jb) {
+            piv[j0 + k] = j0 + p;
+            if (zero)
+                atomicMin(reinterpret_cast<unsigned long long*>(first_zero),
+                          (unsigned long long)(j0 + k + 1));
+        }
+        Z u[NB];
+        static_for<k, NB>([&](auto cc) __attribute__((always_inline)) {
+            u[decltype(cc)::value] = row_bcast_z<decltype(cc)::value>(uv);
+        });
+        static_for<0, RPT>([&](auto q_) __attribute__((always_inline)) {
+            constexpr int q = decltype(q_)::value;
+            if (zero && !used[q]) row[q][k].x = row[q][k].y = R(0);
+            const bool isp = !used[q] && pos[q] == p;
+            if (!used[q] && pos[q] == k) pos[q] = p;
+            if (isp) pos[q] = k;
+            used[q] = used[q] || isp;
+            if (!used[q] && !zero) {
+                const Z l = cmul(row[q][k], u[k]);
+                row[q][k] = l;
+                static_for<k + 1, NB>([&](auto cc) __attribute__((always_inline)) {
+                    constexpr int c = decltype(cc)::value;
+                    csubmul(row[q][c], l, u[c]);
+                });
+            }
+        });
+    });
+    static_for<0, RPT>([&](auto q_) __attribute__((always_inline)) {
+        constexpr int q = decltype(q_)::value;
+        const int r = t + q * ZN_NTH;
+        if (r >= m) return;
+        from[pos[q]] = r;
+#pragma unroll
+        for (int c = 0; c < NB; ++c)
+            if (c < jb) A[pos[q] + c * lda] = row[q][c];
+    });
+}
+
+constexpr int ZU_CW = 8;                 // columns per workgroup of the update
+
+// The columns right of a panel of NB columns at j0: interchanges, U12 =
+// L11^-1 A12 and A22 -= L21 U12.
+template <typename R, int NB>
+__global__ void __launch_bounds__(256)
+znupdate_kernel(i64 n, typename CplxT<R>::type* __restrict__ Ag, i64 lda, i64 j0,
+                const int* __restrict__ from)
+{
+    typedef typename CplxT<R>::type Z;
+    __shared__ __attribute__((aligned(16))) Z s_u[ZU_CW][16];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, li = lane & 15, g = lane >> 4;
+    const int m = (int)(n - j0);
+    const i64 c0 = j0 + NB + (i64)blockIdx.x * ZU_CW;
+    const int nc = n - c0 < ZU_CW ? (int)(n - c0) : ZU_CW;
+    Z* __restrict__ A = Ag + j0;
+    const Z* __restrict__ L = A + j0 * lda;
+    if (wave < 2) {
+        // column 4 wave + g, row li
+        const int c = 4 * wave + g;
+        const bool in = c < nc && li < NB;
+        Z x, l[NB];
+        x.x = x.y = R(0);
+        if (in) x = A[from[li] + (c0 + c) * lda];
+#pragma unroll
+        for (int k = 0; k < NB; ++k) {
+            l[k].x = l[k].y = R(0);
+            if (li > k && li < NB) l[k] = L[li + k * lda];
+        }
+        static_for<0, NB>([&](auto kc) __attribute__((always_inline)) {
+            constexpr int k = decltype(kc)::value;
+            const Z xk = row_bcast_z<k>(x);
+            if (li > k) csubmul(x, l[k], xk);
+        });
+        s_u[c][li] = x;
+    }
+    __syncthreads();
+    for (int r0 = NB + 64 * wave; r0 < m; r0 += 256) {
+        const int r = r0 + lane, rc = r < m ? r : m - 1, fr = from[rc];
+        Z l[NB], x[ZU_CW];
+#pragma unroll
+        for (int k = 0; k < NB; ++k) l[k] = L[rc + k * lda];
+#pragma unroll
+        for (int c = 0; c < ZU_CW; ++c) x[c] = A[fr + (c0 + (c < nc ? c : nc - 1)) * lda];
+#pragma unroll
+        for (int c = 0; c < ZU_CW; ++c) {
+            const Z uv = s_u[c][li];
+            const R nux = -uv.x, nuy = -uv.y;
+            static_for<0, NB / 4>([&](auto kc) __attribute__((always_inline)) {
+                zbcast_fma4<4 * decltype(kc)::value>(x[c].x, x[c].y, nux, nuy, uv.y, l);
+            });
+        }
+        if (r < m) {
+#pragma unroll
+            for (int c = 0; c < ZU_CW; ++c)
+                if (c < nc) A[r + (c0 + c) * lda] = x[c];
+        }
+    }
+    __syncthreads();
+    // U12 over the old top rows, which the update has taken by now
+    if (t < 16 * ZU_CW) {
+        const int c = t >> 4, k = t & 15;
+        if (c < nc && k < NB) A[k + (c0 + c) * lda] = s_u[c][k];
+    }
+}
+
+// The interchanges of the rows [jn, n) (at most ZN_MMAX of them) that columns
+// [cbeg, cend) still lack: those from the end of the column's panel (of ncol
+// columns) or from jn on.  Row i takes the row that the interchanges, taken
+// backwards, trace it to.  A workgroup per panel.
+template <typename R>
+__global__ void __launch_bounds__(ZN_NTH)
+znleft_kernel(i64 n, typename CplxT<R>::type* __restrict__ A, i64 lda, i64 jn, i64 cbeg, i64 cend,
+              int ncol, const i64* __restrict__ piv)
+{
+    typedef typename CplxT<R>::type Z;
+    constexpr int RPT = (int)(ZN_MMAX / ZN_NTH);
+    __shared__ short s_piv[ZN_MMAX];
+    const int t = threadIdx.x, m = (int)(n - jn);
+    const i64 c0 = cbeg + (i64)blockIdx.x * ncol, c1 = c0 + ncol < cend ? c0 + ncol : cend;
+    const int k0 = c1 > jn ? (int)(c1 - jn) : 0;
+    for (int i = t; i < m; i += ZN_NTH) s_piv[i] = (short)(piv[jn + i] - jn);
+    __syncthreads();
+    int src[RPT];
+#pragma unroll
+    for (int q = 0; q < RPT; ++q) src[q] = t + q * ZN_NTH;
+    for (int k = m - 1; k >= k0; --k) {
+        const int p = s_piv[k];
+#pragma unroll
+        for (int q = 0; q < RPT; ++q) src[q] = src[q] == k ? p : src[q] == p ? k : src[q];
+    }
+    for (i64 c = c0; c < c1; ++c) {
+        Z* a = A + jn + c * lda;
+        Z x[RPT];
+#pragma unroll
+        for (int q = 0; q < RPT; ++q) {
+            x[q].x = x[q].y = R(0);
+            if (t + q * ZN_NTH < m) x[q] = a[src[q]];
+        }
+        __syncthreads();                             // every load before any store
+#pragma unroll
+        for (int q = 0; q < RPT; ++q)
+            if (t + q * ZN_NTH < m && src[q] != t + q * ZN_NTH) a[t + q * ZN_NTH] = x[q];
+    }
+}
+
+// Factor rows and columns [jn, n), n - jn <= ZN_MMAX, and give the columns
+// left of jn their interchanges.  from: n ints.
+template <typename R>
+int zgetrf_tail(i64 n, typename CplxT<R>::type* A, i64 lda, i64 jn, i64* piv, i64* d_fz, int* from,
+                hipStream_t s)
+{
+    // the panel width follows the rows a thread holds (registers)
+    i64 jw = n;                              // the first wide panel
+    for (i64 j0 = jn; j0 < n;) {
+        const i64 m = n - j0;
+        const int nb = m > 2 * ZN_NTH ? 8 : 16;
+        if (nb == 16 && jw == n) jw = j0;
+        const int jb = (int)(m < nb ? m : nb);
+#define ZN_PANEL(RPT, NB)                                                                      \
+    hipLaunchKernelGGL((znpanel_kernel<R, RPT, NB>), dim3(1), dim3(ZN_NTH), 0, s, n, A, lda,   \
+                       j0, jb, piv, d_fz, from)
+        if (m > 2 * ZN_NTH) ZN_PANEL(4, 8);
+        else if (m > ZN_NTH) ZN_PANEL(2, 16);
+        else ZN_PANEL(1, 16);
+#undef ZN_PANEL
+        const i64 right = n - j0 - nb;
+        if (right > 0) {
+            const dim3 grid((unsigned)((right + ZU_CW - 1) / ZU_CW));
+            if (nb == 8)
+                hipLaunchKernelGGL((znupdate_kernel<R, 8>), grid, dim3(256), 0, s, n, A, lda, j0,
+                                   from);
+            else
+                hipLaunchKernelGGL((znupdate_kernel<R, 16>), grid, dim3(256), 0, s, n, A, lda, j0,
+                                   from);
+        }
+        TMVX_CHECK_LAUNCH();
+        j0 += jb;
+    }
+    auto left = [&](i64 cbeg, i64 cend, int ncol) {
+        if (cend > cbeg)
+            hipLaunchKernelGGL(znleft_kernel<R>, dim3((unsigned)((cend - cbeg + ncol - 1) / ncol)),
+                               dim3(ZN_NTH), 0, s, n, A, lda, jn, cbeg, cend, ncol, piv);
+    };
+    left(0, jn, 16);
+    left(jn, jw, 8);
+    left(jw, n, 16);
+    return hip_status(hipGetLastError());
+}
+
 template <typename R>
 int zgetrf_impl(i64 n, R* Ar, i64 lda, i64* piv, i64* info, hipStream_t s)
 {
@@ -173,19 +510,23 @@ int zgetrf_impl(i64 n, R* Ar, i64 lda, i64* piv, i64* info, hipStream_t s)
     if (!Ar || !piv) return TMVX_ERR_ARG;
     if (reinterpret_cast<uintptr_t>(Ar) % sizeof(Z)) return TMVX_ERR_ARG;
     Z* A = reinterpret_cast<Z*>(Ar);
-    i64* d_fz = nullptr;
-    if (hipMallocAsync((void**)&d_fz, sizeof(i64), s) != hipSuccess) return TMVX_ERR_ALLOC;
+    i64* d_fz = nullptr;                     // the first zero pivot, then zgetrf_tail's row map
+    if (hipMallocAsync((void**)&d_fz, sizeof(i64) + sizeof(int) * ZN_MMAX, s) != hipSuccess)
+        return TMVX_ERR_ALLOC;
     const i64 big = n + 1;
     hipLaunchKernelGGL(set_i64_kernel, dim3(1), dim3(1), 0, s, d_fz, big);
     int rc = hip_status(hipGetLastError());
     for (i64 j0 = 0; j0 < n && rc == TMVX_OK; j0 += ZP_NB) {
-        const int jb = (int)(n - j0 < ZP_NB ? n - j0 : ZP_NB);
+        if (n - j0 <= ZN_MMAX) {
+            rc = zgetrf_tail<R>(n, A, lda, j0, piv, d_fz, reinterpret_cast<int*>(d_fz + 1), s);
+            break;
+        }
+        const int jb = ZP_NB;
         const i64 j1 = j0 + jb;
         hipLaunchKernelGGL(zpanel_kernel<R>, dim3(1), dim3(ZP_NTH), 0, s, n, A, lda, j0, j1, piv,
                            d_fz);
         if ((rc = hip_status(hipGetLastError())) != TMVX_OK) break;
         const i64 nr = n - j1;
-        if (nr <= 0) break;
         hipLaunchKernelGGL(ztrsm_u12_kernel<R>, dim3((unsigned)((nr + 255) / 256)), dim3(256), 0, s,
                            n, A, lda, j0, jb, j1);
         if ((rc = hip_status(hipGetLastError())) != TMVX_OK) break;
@@ -278,6 +619,108 @@ zsweep_kernel(i64 n, const typename CplxT<R>::type* __restrict__ LU, i64 lda,
     }
 }
 
+// One right-hand side per workgroup, n <= ZS_NMAX: both triangular solves on
+// the vector in LDS.  Blocks of 16 rows: a thread loads its row's 16 entries of
+// the block's columns, the first wave meanwhile solves the block (a row per
+// lane, solved entries by DPP broadcast, one division an entry), then every row
+// to come takes the block's product.  Bound: the block's chain of 16 divisions
+// and one barrier pair per block.  mode as in zsweep_kernel; perm: row i of P A
+// is row perm[i] of A.
+constexpr int ZS_NMAX = 4096;
+constexpr int ZS_NTH = 512;
+
+template <typename R, int MODE>
+__device__ __forceinline__ void zsolve_sweep(int n, const typename CplxT<R>::type* __restrict__ LU,
+                                             i64 lda, typename CplxT<R>::type* s_b,
+                                             int* __restrict__ singular)
+{
+    typedef typename CplxT<R>::type Z;
+    constexpr bool fwd = MODE == 0 || MODE == 2, diag = MODE == 1 || MODE == 2;
+    const int t = threadIdx.x, lane = t & 63, li = lane & 15;
+    const int nb = (n + 15) >> 4;
+    Z zero;
+    zero.x = zero.y = R(0);
+    // op(A)(i, 16 b + k), k < 16; columns past n and rows past the end as 0
+    auto load = [&](int i, int b, Z (&a)[16]) __attribute__((always_inline)) {
+        static_for<0, 16>([&](auto kc) __attribute__((always_inline)) {
+            constexpr int k = decltype(kc)::value;
+            const int c = 16 * b + k;
+            a[k] = zero;
+            if (i >= 0 && i < n && c < n) a[k] = MODE < 2 ? LU[i + c * lda] : LU[c + i * lda];
+        });
+    };
+    for (int q = 0; q < nb; ++q) {
+        const int b = fwd ? q : nb - 1 - q;
+        // rows to come: [r0, r1)
+        const int r0 = fwd ? 16 * (b + 1) : 0, r1 = fwd ? n : 16 * b;
+        Z a[16];
+        load(r0 + t < r1 ? r0 + t : -1, b, a);
+        if (t < 64) {
+            const int r = 16 * b + li;
+            Z x = r < n ? s_b[r] : zero, d[16], dd = zero;
+            load(r, b, d);
+            if constexpr (diag) {
+                static_for<0, 16>([&](auto kc) __attribute__((always_inline)) {
+                    constexpr int k = decltype(kc)::value;
+                    if (li == k) dd = d[k];
+                });
+            }
+            const bool dz = diag && r < n && dd.x == R(0) && dd.y == R(0);
+            static_for<0, 16>([&](auto qc) __attribute__((always_inline)) {
+                constexpr int k = fwd ? decltype(qc)::value : 15 - decltype(qc)::value;
+                if constexpr (diag) {
+                    if (li == k && r < n) {
+                        if (dz) {
+                            if (x.x != R(0) || x.y != R(0)) *singular = 1;
+                            x = zero;
+                        } else {
+                            x = cdiv(x, dd);
+                        }
+                    }
+                }
+                const Z xk = row_bcast_z<k>(x);
+                if (fwd ? li > k : li < k) csubmul(x, d[k], xk);
+            });
+            if (lane < 16 && r < n) s_b[r] = x;
+        }
+        __syncthreads();
+        const Z xv = 16 * b + li < n ? s_b[16 * b + li] : zero;
+        for (int i0 = r0; i0 < r1; i0 += ZS_NTH) {
+            const int i = i0 + t;
+            if (i0 > r0) load(i < r1 ? i : -1, b, a);
+            Z x = i < r1 ? s_b[i] : zero;
+            static_for<0, 16>([&](auto kc) __attribute__((always_inline)) {
+                constexpr int k = decltype(kc)::value;
+                csubmul(x, a[k], row_bcast_z<k>(xv));
+            });
+            if (i < r1) s_b[i] = x;
+        }
+        __syncthreads();
+    }
+}
+
+template <typename R>
+__global__ void __launch_bounds__(ZS_NTH)
+zsolve_kernel(int trans, int n, const typename CplxT<R>::type* __restrict__ LU, i64 lda,
+              const i64* __restrict__ perm, typename CplxT<R>::type* __restrict__ B, i64 ldb,
+              int* __restrict__ singular)
+{
+    typedef typename CplxT<R>::type Z;
+    __shared__ __attribute__((aligned(16))) Z s_b[ZS_NMAX];
+    Z* b = B + (i64)blockIdx.x * ldb;
+    const int t = threadIdx.x;
+    for (int i = t; i < n; i += ZS_NTH) s_b[i] = trans ? b[i] : b[perm[i]];
+    __syncthreads();
+    if (!trans) {
+        zsolve_sweep<R, 0>(n, LU, lda, s_b, singular);
+        zsolve_sweep<R, 1>(n, LU, lda, s_b, singular);
+    } else {
+        zsolve_sweep<R, 2>(n, LU, lda, s_b, singular);
+        zsolve_sweep<R, 3>(n, LU, lda, s_b, singular);
+    }
+    for (int i = t; i < n; i += ZS_NTH) b[trans ? perm[i] : i] = s_b[i];
+}
+
 template <typename R>
 int zgetrs_impl(int trans, i64 n, i64 nrhs, const R* LUr, i64 lda, const i64* piv, R* Br, i64 ldb,
                 hipStream_t s)
@@ -291,12 +734,23 @@ int zgetrs_impl(int trans, i64 n, i64 nrhs, const R* LUr, i64 lda, const i64* pi
     if (nrhs > 0x7fffffff) return TMVX_ERR_UNSUPPORTED;
     const Z* LU = reinterpret_cast<const Z*>(LUr);
     Z* B = reinterpret_cast<Z*>(Br);
-    int* d_sing = nullptr;
-    if (hipMallocAsync((void**)&d_sing, sizeof(int), s) != hipSuccess) return TMVX_ERR_ALLOC;
+    const bool in_lds = n <= ZS_NMAX;
+    int* d_sing = nullptr;                   // the flag, then (n <= ZS_NMAX) the permutation
+    if (hipMallocAsync((void**)&d_sing, 16 + (in_lds ? sizeof(i64) * (size_t)n : 0), s) !=
+        hipSuccess)
+        return TMVX_ERR_ALLOC;
     hipLaunchKernelGGL(set_int_kernel, dim3(1), dim3(1), 0, s, d_sing, 0);
     int rc = hip_status(hipGetLastError());
     const dim3 gp((unsigned)((nrhs + 63) / 64)), bp(64), gs((unsigned)nrhs), bs(256);
-    if (rc == TMVX_OK && !trans) {
+    if (rc == TMVX_OK && in_lds) {
+        i64* perm = reinterpret_cast<i64*>(reinterpret_cast<char*>(d_sing) + 16);
+        rc = piv_to_perm(n, piv, perm, s);
+        if (rc == TMVX_OK) {
+            hipLaunchKernelGGL(zsolve_kernel<R>, gs, dim3(ZS_NTH), 0, s, trans, (int)n, LU, lda,
+                               perm, B, ldb, d_sing);
+            rc = hip_status(hipGetLastError());
+        }
+    } else if (rc == TMVX_OK && !trans) {
         hipLaunchKernelGGL(zpermute_kernel<R>, gp, bp, 0, s, n, nrhs, B, ldb, piv, 0);
         hipLaunchKernelGGL(zsweep_kernel<R>, gs, bs, 0, s, n, LU, lda, B, ldb, 0, d_sing);
         hipLaunchKernelGGL(zsweep_kernel<R>, gs, bs, 0, s, n, LU, lda, B, ldb, 1, d_sing);
