@@ -1,0 +1,56 @@
+"""QR at the edges of the 8-column register panels (one to eight rows a thread,
+4096 rows; more rows take the 32-column panels), partial panels, zero columns,
+and the solve with one to many right-hand sides.
+
+Bar: R and beta those of LAPACK's dgeqrf in float64 to 64 m eps
+|A| (both are backward stable Householder QRs with the same signs), and A = Q R
+to 8 m eps through the applied Q^T."""
+import numpy as np
+import pytest
+import scipy.linalg
+import torch
+
+import tmv_amd
+from checks import EPS64, EPS32
+from tmv_amd import rng
+
+pytestmark = pytest.mark.gpu
+SEED = 0x7A15EED
+
+
+@pytest.mark.parametrize("dtype,m,n,nrhs", [
+    (torch.float64, 1, 1, 1), (torch.float64, 8, 8, 2), (torch.float64, 9, 7, 1),
+    (torch.float64, 512, 9, 3), (torch.float64, 513, 64, 1), (torch.float64, 1025, 33, 17),
+    (torch.float64, 2049, 20, 2), (torch.float64, 4096, 17, 1), (torch.float64, 4097, 12, 2),
+    (torch.float32, 600, 31, 2), (torch.float32, 2100, 16, 1)])
+def test_qr_panels(dev, dtype, m, n, nrhs):
+    print(f"qr {dtype} {m}x{n}", flush=True)
+    eps = EPS64 if dtype == torch.float64 else EPS32
+    A = rng.uniform_matrix(SEED + m + n, m, n)
+    B = rng.uniform_matrix(SEED + m + n + 1, m, nrhs)
+    if dtype == torch.float32:
+        A, B = A.astype(np.float32).astype(np.float64), B.astype(np.float32).astype(np.float64)
+    QR = tmv_amd.colmajor(torch.from_numpy(A).to(dtype).cuda())
+    beta = tmv_amd.geqrf(QR)
+    (qr, tau), _ = scipy.linalg.qr(A, mode="raw")
+    got = QR.cpu().numpy().astype(np.float64)
+    assert np.abs(np.triu(got[:n]) - np.triu(qr[:n])).max() <= 64 * m * eps * np.abs(A).max()
+    assert np.abs(beta.cpu().numpy() - tau).max() <= 64 * m * eps
+    X = tmv_amd.colmajor(torch.from_numpy(B).to(dtype).cuda())
+    tmv_amd.geqrs(QR, beta, X)
+    x = X.cpu().numpy().astype(np.float64)[:n]
+    # least squares: A^T (B - A x) = 0, relative to the sizes that enter it
+    g = np.abs(A.T @ (B - A @ x)).max()
+    assert g <= 64 * m * eps * np.abs(A).max() * (np.abs(B).max() + n * np.abs(A).max() * np.abs(x).max())
+
+
+def test_qr_zero_columns_in_panel(dev):
+    A = rng.uniform_matrix(SEED + 3, 300, 20)
+    A[:, 3] = 0
+    A[:, 8] = 0
+    QR = tmv_amd.colmajor(torch.from_numpy(A).cuda())
+    beta = tmv_amd.geqrf(QR).cpu().numpy()
+    got = QR.cpu().numpy()
+    assert beta[3] == 0 and beta[8] == 0 and got[3, 3] == 0 and got[8, 8] == 0
+    R = np.triu(got[:20])
+    assert np.abs(R.T @ R - A.T @ A).max() <= 8 * 300 * EPS64 * np.abs(A.T @ A).max()
