@@ -10,8 +10,8 @@
 //
 // Per panel of NB columns starting at j0:
 //   1. panel_kernel: G workgroups each hold a contiguous slab of the panel's
-//      rows in registers (one row per thread, kept rotated so the current
-//      column is always register 0).  Per column: local argmax (largest
+//      rows in registers (one row per thread, rotated by blocks of 8
+//      columns).  Per column: local argmax (largest
 //      |a|, lowest row on ties, as TMV's strict '>'); each workgroup
 //      publishes its candidate row, value and index to its slot as tagged
 //      64-bit words (32 payload bits + the global column number), and every
@@ -163,16 +163,22 @@ __device__ long long g_panel_trace_j0;
 // block values) per workgroup.  Operation order per element is that of the
 // unblocked right-looking elimination, so the factors do not depend on BB.
 //
-// Registers hold the row rotated: by whole blocks at block ends (before
-// block kb, row[c] is panel column (kb*BB + c) mod NB for c >= BB), and
-// within the block by one column per step (the current column is always
-// row[0]), so the column loop is one copy of code with static register
-// indices.
+// Registers hold the row rotated by whole blocks at block ends (before block
+// kb, row[c] is panel column (kb*BB + c) mod NB), so the block loop is one copy
+// of code with static register indices; within the block the columns are
+// unrolled (rotating the row by a column per step cost BB register moves of the
+// loop's carried values each).
 //
-// Per column: each wave's argmax goes to LDS (double-buffered by column
-// parity), one barrier, wave 0 reduces them, publishes the workgroup's
-// candidate, receives every workgroup's slot (lane q holds slot q), picks
-// the winner and puts it in LDS; a second barrier hands it to every wave.
+// Per column: each wave's candidate (the search on integer keys) goes to LDS
+// (double-buffered by column parity), one barrier.  One workgroup (SOLO): every
+// wave reduces the candidates itself and reads the winner's values where they
+// lie.  Several: wave 0 reduces them, publishes the workgroup's candidate,
+// receives every workgroup's slot (lane q holds slot q), picks the winner and
+// puts it in LDS; a second barrier hands it to every wave.
+// Bound: the chain of a column.  FP64, 64 columns, 512 rows: 122 -> 69 us (one
+// barrier instead of two, keys instead of FP64 maxima, no row rotation); with
+// the exchange 3.4 -> 2.5 us a column at 8192 rows, whose floor is the round
+// trip through the device's coherence point.
 template <typename T, int NB, int BB, int NTH, bool SOLO>
 __global__ void __launch_bounds__(NTH)
 panel_kernel(T* __restrict__ A, i64 lda, i64 n, i64 j0, int jb, i64* __restrict__ piv,
@@ -191,14 +197,10 @@ panel_kernel(T* __restrict__ A, i64 lda, i64 n, i64 j0, int jb, i64* __restrict_
     const int r = w * NTH + t;                   // panel-relative row
     const bool own = r < m;
 
-    __shared__ T s_wv[2][NW];                    // per-wave candidates (column parity)
-    __shared__ int s_wi[2][NW];
+    __shared__ int4 s_cand[2][NW];               // per-wave candidates (column parity)
     __shared__ __attribute__((aligned(16))) T s_wrow[2][NW][BB];   // their block values
     __shared__ __attribute__((aligned(16))) T s_pv[BB];            // the pivot row's block values
-    __shared__ int s_p, s_zero, s_fail;
-    // the panel's interchange list, written out at the end: a global store
-    // in the column loop would make the next barrier wait for it
-    __shared__ int s_piv[NB];
+    __shared__ int s_win, s_fail;
     __shared__ int s_own[BB];                    // block pivot i is held here
     // block pivot rows (block order), as 32-bit words: staged by their
     // owners or received; U12 is solved in place in columns >= BB
@@ -217,6 +219,8 @@ panel_kernel(T* __restrict__ A, i64 lda, i64 n, i64 j0, int jb, i64* __restrict_
     }
     int pos = r;                  // current position (panel-relative)
     bool used = !own;             // a pivot row (or no row at all)
+    int mypk = 0;                 // thread k: pivot of column k (stored at the end: a global
+                                  // store in the column loop would be waited for)
     int mypiv = -1;               // index of this row among the current block's pivots
     bool dfr = false;             // takes the previous block's deferred update chunks
     int nchunk = 0;               // deferred chunks pending (uniform)
@@ -235,41 +239,38 @@ panel_kernel(T* __restrict__ A, i64 lda, i64 n, i64 j0, int jb, i64* __restrict_
         for (int q = 0; q < BB; ++q) row[NB - BB + q] = first[q];
         ++nrot;
     };
-    auto rotate_in_block = [&]() __attribute__((always_inline)) {
-        const T first = row[0];
-#pragma unroll
-        for (int q = 0; q < BB - 1; ++q) row[q] = row[q + 1];
-        row[BB - 1] = first;
-    };
     // Deferred share of the previous block's rank-BB update: chunk j (the
     // BB columns now at row[j*BB ..]) with the block's multipliers (now at
     // row[NB-BB ..]) and its U12 rows (still in s_rows, columns (j+1)*BB ..).
     // Applied while the workgroup waits for the exchange, chunk j at column
     // step (j - 1) mod BB (one chunk per step for NB = 64, up to two for
     // NB = 128); all are done before the block's own end.
-    auto deferred_chunk = [&](int kk) __attribute__((always_inline)) {
+    auto deferred_chunk = [&](auto kc) __attribute__((always_inline)) {
+        constexpr int kk = decltype(kc)::value;
         if (!dfr) return;
         typedef typename Vec16<T>::type VT;
         constexpr int VN = Vec16<T>::n;
         static_assert(NBLK - 2 <= 2 * BB, "two chunks per step at most");
-        static_for<1, NBLK - 1>([&](auto jc) {
+        static_for<1, NBLK - 1>([&](auto jc) __attribute__((always_inline)) {
             constexpr int j = decltype(jc)::value;
-            if ((j - 1) % BB != kk || j > nchunk) return;             // uniform
-            static_for<0, BB>([&](auto ic) {
-                constexpr int i = decltype(ic)::value;
-                const T li = row[NB - BB + i];
-                static_for<0, BB / VN>([&](auto qc) {
-                    constexpr int q = decltype(qc)::value * VN;
-                    const VT u = *reinterpret_cast<const VT*>(&s_rows[i][(j + 1) * BB + q]);
-                    static_for<0, VN>([&](auto uc) {
-                        constexpr int x = decltype(uc)::value;
-                        row[j * BB + q + x] -= li * u[x];
+            if constexpr ((j - 1) % BB == kk) {
+                if (j > nchunk) return;                               // uniform
+                static_for<0, BB>([&](auto ic) __attribute__((always_inline)) {
+                    constexpr int i = decltype(ic)::value;
+                    const T li = row[NB - BB + i];
+                    static_for<0, BB / VN>([&](auto qc) __attribute__((always_inline)) {
+                        constexpr int q = decltype(qc)::value * VN;
+                        const VT u = *reinterpret_cast<const VT*>(&s_rows[i][(j + 1) * BB + q]);
+                        static_for<0, VN>([&](auto uc) __attribute__((always_inline)) {
+                            constexpr int x = decltype(uc)::value;
+                            row[j * BB + q + x] -= li * u[x];
+                        });
                     });
                 });
-            });
-            // keeps the per-chunk branches apart: merged, they would index
-            // row[] with the runtime chunk number and move it to memory
-            __asm__ volatile("" ::: "memory");
+                // keeps the branches apart: merged, they would index row[]
+                // with the runtime chunk number and move it to memory
+                __asm__ volatile("" ::: "memory");
+            }
         });
     };
     // Bounded wait bookkeeping: false once the wait has to give up --
@@ -290,91 +291,93 @@ panel_kernel(T* __restrict__ A, i64 lda, i64 n, i64 j0, int jb, i64* __restrict_
     for (int kb = 0; kb < nblk && alive; ++kb) {
         const int c0 = kb * BB;
         const int bcnt = (jb - c0) < BB ? (jb - c0) : BB;
-        int kk = 0;
-        for (; kk < bcnt; ++kk) {
+        static_for<0, BB>([&](auto kc) __attribute__((always_inline)) {
+            constexpr int kk = decltype(kc)::value;
+            if (!alive || kk >= bcnt) return;                        // uniform
+            typedef typename Vec16<T>::type VT;
+            constexpr int VN = Vec16<T>::n;
             const int k = c0 + kk;
             const int par = k & 1;
-            const unsigned tag32 = (unsigned)(j0 + k + 1);
-            const unsigned long long tag = (unsigned long long)tag32 << 32;
-            // -- wave argmax over the unused rows ---------------------------
-            T v;
-            int vi;
-            lanes_argmax<64>(used ? T(-1) : fabs(row[0]), pos, v, vi);
-            if (lane == 0) { s_wv[par][wave] = v; s_wi[par][wave] = vi; }
-            if (!used && pos == vi) {
-                typedef typename Vec16<T>::type VT;
-                constexpr int VN = Vec16<T>::n;
-                static_for<0, BB / VN>([&](auto qc) {
+            // -- wave candidate over the unused rows ------------------------
+            const unsigned khi = used ? 0u : mag_hi(row[kk]), klo = mag_lo(row[kk]);
+            unsigned mk;
+            if (lane == lanes_best<64, T>(khi, klo, pos, mk)) {
+                s_cand[par][wave] = make_int4((int)khi, (int)klo, pos, 0);
+                static_for<kk / VN, BB / VN>([&](auto qc) __attribute__((always_inline)) {
                     constexpr int q = decltype(qc)::value * VN;
                     VT x;
-                    static_for<0, VN>([&](auto uc) { x[decltype(uc)::value] = row[q + decltype(uc)::value]; });
+                    static_for<0, VN>([&](auto uc) __attribute__((always_inline)) {
+                        x[decltype(uc)::value] = row[q + decltype(uc)::value];
+                    });
                     *reinterpret_cast<VT*>(&s_wrow[par][wave][q]) = x;
                 });
             }
             __syncthreads();
             PANEL_TRACE(k, 0);
-            if (wave != 0) deferred_chunk(kk);     // inside the exchange wait
-            if (wave == 0) {
-                // -- this workgroup's candidate, published as tagged words;
-                //    word f of workgroup q lives at cs[f * G + q] ----------
-                unsigned long long* cs = wk.cslots + (i64)par * CS::SIZE * G;
-                const int myi = lane < NW ? s_wi[par][lane] : INT_MAX;
-                T bv;
-                int bi;
-                lanes_argmax<8>(lane < NW ? s_wv[par][lane] : T(-1), myi, bv, bi);
-                const unsigned long long hw = __ballot(lane < NW && myi == bi);
-                const int ww = hw ? (int)__builtin_ctzll(hw) : 0;
-                if (!SOLO && lane < CS::SIZE) {
-                    const int e = lane >= CS::ROW ? lane - CS::ROW : 0;
-                    const unsigned rowpay = half_bits(s_wrow[par][ww][e / WPV], e % WPV);
-                    const unsigned pay = lane < CS::POS ? half_bits(bv, lane)
-                                       : lane == CS::POS ? (unsigned)bi : rowpay;
-                    cstore(cs + (i64)lane * G + w, tag | pay);
-                }
-                PANEL_TRACE(k, 1);
-                deferred_chunk(kk);                // before any slot can arrive
-                // -- receive every slot: lane q holds slot q ----------------
-                T bestv = T(-1);
-                int besti = INT_MAX;
-                unsigned bpay[BW];
-#pragma unroll
-                for (int f = 0; f < BW; ++f) bpay[f] = 0u;
-                bool ok = true;
-                auto take = [&](const unsigned long long (&wv)[CS::SIZE], bool valid)
-                    __attribute__((always_inline)) {
-                    if (!valid) return;
-                    unsigned pay[CS::SIZE];
-#pragma unroll
-                    for (int f = 0; f < CS::SIZE; ++f) pay[f] = (unsigned)wv[f];
-                    const T qv = from_halves<T>(&pay[CS::VAL]);
-                    const int qi = (int)pay[CS::POS];
-                    if (better(qv, qi, bestv, besti)) {
-                        bestv = qv;
-                        besti = qi;
-#pragma unroll
-                        for (int f = 0; f < BW; ++f) bpay[f] = pay[CS::ROW + f];
+            int p;                                   // pivot position, -1: none
+            const T* pr;                             // the pivot row's block values
+            if constexpr (SOLO) {
+                // one workgroup holds every row: each wave picks the winner
+                // among the waves' candidates itself
+                const int4 c = s_cand[par][lane < NW ? lane : 0];
+                const int ww = lanes_best<8, T>(lane < NW ? (unsigned)c.x : 0u, (unsigned)c.y, c.z, mk);
+                p = mk < mag_tiny<T>() ? -1 : __builtin_amdgcn_readlane(c.z, ww);
+                pr = s_wrow[par][ww];
+                PANEL_TRACE(k, 2);
+                if (p < 0 && t == 0)
+                    atomicMin(reinterpret_cast<unsigned long long*>(wk.first_zero),
+                              (unsigned long long)(j0 + k + 1));
+            } else {
+                if (wave != 0) deferred_chunk(kc);   // inside the exchange wait
+                if (wave == 0) {
+                    // -- this workgroup's candidate, published as tagged
+                    //    words; word f of workgroup q lives at cs[f * G + q]
+                    const unsigned tag32 = (unsigned)(j0 + k + 1);
+                    const unsigned long long tag = (unsigned long long)tag32 << 32;
+                    unsigned long long* cs = wk.cslots + (i64)par * CS::SIZE * G;
+                    const int4 c = s_cand[par][lane < NW ? lane : 0];
+                    const int ww = lanes_best<8, T>(lane < NW ? (unsigned)c.x : 0u, (unsigned)c.y,
+                                                    c.z, mk);
+                    if (lane < CS::SIZE) {
+                        // s_cand as words: high key, low word, position
+                        const int e = lane >= CS::ROW ? lane - CS::ROW : 0;
+                        const unsigned rowpay =
+                            reinterpret_cast<const unsigned*>(s_wrow[par][ww])[e];
+                        const unsigned kpay = reinterpret_cast<const unsigned*>(
+                            &s_cand[par][ww])[lane < CS::POS ? CS::POS - 1 - lane : 2];
+                        cstore(cs + (i64)lane * G + w, tag | (lane < CS::ROW ? kpay : rowpay));
                     }
-                };
-                auto complete = [&](const unsigned long long (&wv)[CS::SIZE], bool valid)
-                    __attribute__((always_inline)) -> bool {
-                    bool have = true;
-                    static_for<0, CS::SIZE>([&](auto fc) {
-                        constexpr int f = decltype(fc)::value;
-                        have &= (unsigned)(wv[f] >> 32) == tag32;
-                    });
-                    return __ballot(valid && !have) == 0ull;
-                };
-                if constexpr (SOLO) {
-                    // one workgroup holds every row: its candidate is the
-                    // winner, no exchange
-                    if (lane == 0) {
-                        bestv = bv;
-                        besti = bi;
+                    PANEL_TRACE(k, 1);
+                    deferred_chunk(kc);              // before any slot can arrive
+                    // -- receive every slot: lane q holds slot q ------------
+                    unsigned bhi = 0u, blo = 0u;
+                    int bpos = INT_MAX;
+                    unsigned bpay[BW];
 #pragma unroll
-                        for (int f = 0; f < BW; ++f)
-                            bpay[f] = half_bits(s_wrow[par][ww][f / WPV], f % WPV);
-                    }
-                } else {
+                    for (int f = 0; f < BW; ++f) bpay[f] = 0u;
+                    bool ok = true;
+                    auto take = [&](const unsigned long long (&wv)[CS::SIZE], bool valid)
+                        __attribute__((always_inline)) {
+                        const unsigned qhi = valid ? (unsigned)wv[CS::POS - 1] : 0u;
+                        const unsigned qlo = WPV == 2 ? (unsigned)wv[0] : 0u;
+                        const int qi = (int)wv[CS::POS];
+                        if (qhi > bhi || (qhi == bhi && (qlo > blo || (qlo == blo && qi < bpos)))) {
+                            bhi = qhi;
+                            blo = qlo;
+                            bpos = qi;
+#pragma unroll
+                            for (int f = 0; f < BW; ++f) bpay[f] = (unsigned)wv[CS::ROW + f];
+                        }
+                    };
+                    auto complete = [&](const unsigned long long (&wv)[CS::SIZE], bool valid)
+                        __attribute__((always_inline)) -> bool {
+                        bool have = true;
+                        static_for<0, CS::SIZE>([&](auto fc) __attribute__((always_inline)) {
+                            constexpr int f = decltype(fc)::value;
+                            have &= (unsigned)(wv[f] >> 32) == tag32;
+                        });
+                        return __ballot(valid && !have) == 0ull;
+                    };
                     for (int qb = 0; qb < G && ok; qb += 64) {
                         const int q = qb + lane;
                         const bool valid = q < G;
@@ -383,7 +386,7 @@ panel_kernel(T* __restrict__ A, i64 lda, i64 n, i64 j0, int jb, i64* __restrict_
                         unsigned spins = 0;
                         long long t0 = 0;
                         while (true) {
-                            static_for<0, CS::SIZE>([&](auto fc) {
+                            static_for<0, CS::SIZE>([&](auto fc) __attribute__((always_inline)) {
                                 constexpr int f = decltype(fc)::value;
                                 wv[f] = cload(src + (i64)f * G);
                             });
@@ -393,74 +396,63 @@ panel_kernel(T* __restrict__ A, i64 lda, i64 n, i64 j0, int jb, i64* __restrict_
                         }
                         if (ok) take(wv, valid);
                     }
-                }
-                PANEL_TRACE(k, 2);
-                if (ok) {
-                    // -- the global winner (the same in every workgroup) ----
-                    T gv;
-                    int gi;
-                    lanes_argmax<64>(bestv, besti, gv, gi);
-                    const unsigned long long hg = __ballot(besti == gi);
-                    const int wl = hg ? (int)__builtin_ctzll(hg) : 0;
-                    const bool zero = !(gv >= tiny<T>());              // TMV_Underflow
-                    const int p = zero ? k : gi;
-                    // the winner's block values, written by the lane that
-                    // holds them (readlanes would each wait for an SGPR)
+                    PANEL_TRACE(k, 2);
+                    // -- the global winner (the same in every workgroup); its
+                    // block values go to LDS from the lane that holds them
+                    // (readlanes would each wait for an SGPR) -------------
+                    const int wl = lanes_best<64, T>(bhi, blo, bpos, mk);
                     if (lane == wl) {
-                        static_for<0, BB>([&](auto jc) {
-                            constexpr int j = decltype(jc)::value;
-                            s_pv[j] = from_halves<T>(&bpay[j * WPV]);
+                        static_for<kk / VN, BB / VN>([&](auto qc) __attribute__((always_inline)) {
+                            constexpr int q = decltype(qc)::value * VN;
+                            VT x;
+                            static_for<0, VN>([&](auto uc) __attribute__((always_inline)) {
+                                constexpr int u = decltype(uc)::value;
+                                x[u] = from_halves<T>(&bpay[(q + u) * WPV]);
+                            });
+                            *reinterpret_cast<VT*>(&s_pv[q]) = x;
                         });
+                        const bool zero = mk < mag_tiny<T>();        // TMV_Underflow
+                        s_win = !ok ? -2 : zero ? -1 : bpos;
+                        if (ok && zero && w == 0)
+                            atomicMin(reinterpret_cast<unsigned long long*>(wk.first_zero),
+                                      (unsigned long long)(j0 + k + 1));
                     }
-                    if (lane == 0) {
-                        s_zero = zero ? 1 : 0;
-                        s_p = p;
-                        if (w == 0) {
-                            s_piv[k] = p;
-                            if (zero)
-                                atomicMin(reinterpret_cast<unsigned long long*>(wk.first_zero),
-                                          (unsigned long long)(j0 + k + 1));
-                        }
-                    }
-                } else if (lane == 0) {
-                    s_fail = 1;
                 }
+                __syncthreads();
+                p = s_win;
+                pr = s_pv;
+                if (p == -2) { alive = false; return; }              // uniform
             }
-            __syncthreads();
-            if (s_fail) { alive = false; break; }                    // uniform after the barrier
             // -- interchange (positions only) and the block's update ---------
-            const int p = s_p;
-            if (s_zero) {
-                // TMV: zero the column from the diagonal down, interchange
-                // with itself; the row at position k is the pivot row.
-                if (!used) row[0] = T(0);
-                if (!used && pos == k) { used = true; mypiv = kk; }
-            } else {
-                if (!used && pos == p) { used = true; mypiv = kk; pos = k; }
-                else if (!used && pos == k) pos = p;
-                if (!used) {
-                    typedef typename Vec16<T>::type VT;
-                    constexpr int VN = Vec16<T>::n;
-                    T pv[BB];
-                    static_for<0, BB / VN>([&](auto qc) {
-                        constexpr int q = decltype(qc)::value * VN;
-                        const VT x = *reinterpret_cast<const VT*>(&s_pv[q]);
-                        static_for<0, VN>([&](auto uc) { pv[q + decltype(uc)::value] = x[decltype(uc)::value]; });
+            const int pk = p < 0 ? k : p;            // underflow: with itself
+            if (t == k) mypk = pk;
+            // TMV: an underflowing column is zeroed from the diagonal down
+            if (p < 0 && !used) row[kk] = T(0);
+            const bool isp = !used && pos == pk;
+            if (!used && pos == k) pos = pk;
+            if (isp) { used = true; mypiv = kk; pos = k; }
+            if (p >= 0) {
+                T pv[BB];
+                static_for<kk / VN, BB / VN>([&](auto qc) __attribute__((always_inline)) {
+                    constexpr int q = decltype(qc)::value * VN;
+                    const VT x = *reinterpret_cast<const VT*>(pr + q);
+                    static_for<0, VN>([&](auto uc) __attribute__((always_inline)) {
+                        pv[q + decltype(uc)::value] = x[decltype(uc)::value];
                     });
-                    const T l = row[0] * (T(1) / pv[0]);
-                    row[0] = l;
-                    const int lim = BB - kk;       // block columns after this one
-#pragma unroll
-                    for (int c = 1; c < BB; ++c)
-                        if (c < lim) row[c] -= l * pv[c];
+                });
+                const T l = row[kk] * (T(1) / pv[kk]);
+                if (!used) {
+                    row[kk] = l;
+                    static_for<kk + 1, BB>([&](auto cc) __attribute__((always_inline)) {
+                        constexpr int c = decltype(cc)::value;
+                        row[c] -= l * pv[c];
+                    });
                 }
             }
-            rotate_in_block();
+            if constexpr (SOLO) deferred_chunk(kc);  // no wait to hide it in
             PANEL_TRACE(k, 3);
-        }
+        });
         if (!alive) break;
-        // complete the in-block rotation of a partial block
-        for (; kk < BB; ++kk) rotate_in_block();
         if (c0 + BB >= jb) break;
         // -- block end: the BB pivot rows, U12, rank-BB update ---------------
         if (mypiv >= 0) {
@@ -568,7 +560,7 @@ panel_kernel(T* __restrict__ A, i64 lda, i64 n, i64 j0, int jb, i64* __restrict_
     // Restore column order (the rotation is by whole blocks).
     while ((nrot * BB) % NB != 0) rotate_blocks();
     if (!alive) return;
-    if (w == 0 && t < jb) piv[j0 + t] = j0 + s_piv[t];
+    if (w == 0 && t < jb) piv[j0 + t] = j0 + mypk;
     if (!own) return;
     T* dst = A + (j0 + pos) + j0 * lda;
 #pragma unroll
