@@ -17,6 +17,7 @@
 // in MFMA accumulators (16x16 blocks of v_mfma_{f64,f32}_16x16x4).
 #pragma once
 #include "tmvx_gemm_decl.h"
+#include <type_traits>
 
 namespace tmvx {
 
@@ -53,7 +54,7 @@ template <typename Cfg, typename T, bool TA, bool TB>
 __global__ void __launch_bounds__(Cfg::NT) __attribute__((amdgpu_waves_per_eu(Cfg::MINW)))
 gemm_kernel(i64 M, i64 N, i64 K, T alpha, const T* __restrict__ A, i64 lda,
             const T* __restrict__ B, i64 ldb, T beta, T* __restrict__ C,
-            i64 ldc, int vec_ok)
+            i64 ldc)
 {
     constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, WM = Cfg::WM;
     constexpr int NT = Cfg::NT, V = Cfg::V;
@@ -96,38 +97,37 @@ gemm_kernel(i64 M, i64 N, i64 K, T alpha, const T* __restrict__ A, i64 lda,
     };
 
     // ---- global -> registers -------------------------------------------
-    auto load = [&](i64 k0) {
-        const bool fast = vec_ok && full_mn && (k0 + BK <= K);
+    // 16-byte loads need element alignment only (global_load_dwordx4 takes
+    // any dword address), so an odd leading dimension or base takes them too;
+    // a vector that crosses the edge of the matrix is read by element.
+    typedef VT VU __attribute__((aligned(sizeof(T))));
+    auto load_op = [&](const T* X, i64 ld, bool kc, i64 x0, i64 xn, i64 k0, bool fast, int rows,
+                       auto nv, VT* rx) __attribute__((always_inline)) {
 #pragma unroll
-        for (int r = 0; r < Cfg::NVA; ++r) {
+        for (int r = 0; r < decltype(nv)::value; ++r) {
             int x, k;
-            vcoord(t + r * NT, BM, AKC, x, k);
+            vcoord(t + r * NT, rows, kc, x, k);
+            const i64 gx = x0 + x, gk = k0 + k;
+            const T* p = kc ? X + gx * ld + gk : X + gx + gk * ld;
             if (fast) {
-                const T* p = TA ? A + (m0 + x) * lda + (k0 + k) : A + (m0 + x) + (k0 + k) * lda;
-                ra[r] = *reinterpret_cast<const VT*>(p);
+                rx[r] = *reinterpret_cast<const VU*>(p);
             } else {
+                const i64 nx = xn - gx, nkk = K - gk;       // entries left along x and k
+                const i64 along = kc ? nkk : nx, across = kc ? nx : nkk;
+                if (across > 0 && along >= V) {
+                    rx[r] = *reinterpret_cast<const VU*>(p);
+                } else {
 #pragma unroll
-                for (int e = 0; e < V; ++e) {
-                    const i64 gm = m0 + x + (AKC ? 0 : e), gk = k0 + k + (AKC ? e : 0);
-                    ra[r][e] = (gm < M && gk < K) ? (TA ? A[gm * lda + gk] : A[gm + gk * lda]) : T(0);
+                    for (int e = 0; e < V; ++e)
+                        rx[r][e] = (across > 0 && e < along) ? p[e] : T(0);
                 }
             }
         }
-#pragma unroll
-        for (int r = 0; r < Cfg::NVB; ++r) {
-            int x, k;
-            vcoord(t + r * NT, BN, BKC, x, k);
-            if (fast) {
-                const T* p = TB ? B + (k0 + k) * ldb + (n0 + x) : B + (k0 + k) + (n0 + x) * ldb;
-                rb[r] = *reinterpret_cast<const VT*>(p);
-            } else {
-#pragma unroll
-                for (int e = 0; e < V; ++e) {
-                    const i64 gn = n0 + x + (BKC ? 0 : e), gk = k0 + k + (BKC ? e : 0);
-                    rb[r][e] = (gk < K && gn < N) ? (TB ? B[gk * ldb + gn] : B[gk + gn * ldb]) : T(0);
-                }
-            }
-        }
+    };
+    auto load = [&](i64 k0) __attribute__((always_inline)) {
+        const bool fast = full_mn && (k0 + BK <= K);
+        load_op(A, lda, AKC, m0, M, k0, fast, BM, std::integral_constant<int, Cfg::NVA>(), ra);
+        load_op(B, ldb, BKC, n0, N, k0, fast, BN, std::integral_constant<int, Cfg::NVB>(), rb);
     };
 
     // ---- registers -> LDS (same orientation, one 16-byte store each) ----
@@ -221,14 +221,10 @@ int gemm_launch_cfg(int ta, int tb, i64 m, i64 n, i64 k, T alpha, const T* A,
 {
     const i64 tiles = ((m + Cfg::BM - 1) / Cfg::BM) * ((n + Cfg::BN - 1) / Cfg::BN);
     if (tiles > 0x7fffffff) return TMVX_ERR_UNSUPPORTED;
-    const int V = Cfg::V;
-    const int vec_ok =
-        ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) % 16 == 0) &&
-        (lda % V == 0) && (ldb % V == 0);
     dim3 grid((unsigned)tiles), block(Cfg::NT);
 #define TMVX_GEMM_GO(TA_, TB_)                                                 \
     hipLaunchKernelGGL((gemm_kernel<Cfg, T, TA_, TB_>), grid, block, 0, s, m,  \
-                       n, k, alpha, A, lda, B, ldb, beta, C, ldc, vec_ok)
+                       n, k, alpha, A, lda, B, ldb, beta, C, ldc)
     if (!ta && !tb) TMVX_GEMM_GO(false, false);
     else if (!ta && tb) TMVX_GEMM_GO(false, true);
     else if (ta && !tb) TMVX_GEMM_GO(true, false);
