@@ -85,6 +85,11 @@ template <typename T>
 int gemm_launch(int a_rowmajor, int b_rowmajor, i64 m, i64 n, i64 k, T alpha,
                 const T* A, i64 lda, const T* B, i64 ldb, T beta, T* C,
                 i64 ldc, hipStream_t s);
+// The same for a product that runs on a side stream beside a panel chain.
+template <typename T>
+int gemm_launch_beside(int a_rowmajor, int b_rowmajor, i64 m, i64 n, i64 k, T alpha,
+                const T* A, i64 lda, const T* B, i64 ldb, T beta, T* C,
+                i64 ldc, hipStream_t s);
 
 // Complex C := (ar + i ai) op(A) op(B) + (br + i bi) C on interleaved
 // complex storage of real type R (tmvx_complex.hip).

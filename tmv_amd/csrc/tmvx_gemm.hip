@@ -38,24 +38,30 @@ template <> struct GemmTable<float> {
     { switch (cfg) { TMVX_F32_CFGS(TMVX_CFG_NAME) default: return nullptr; } }
 };
 
-// Default configuration by shape (chosen from measurements on MI355X).
-template <typename T> int default_cfg(int ta, int tb, i64 m, i64 n, i64 k);
-// Short K (the LU updates: K = 64 inside an outer panel, K = 256 for the
-// trailing matrix) favours small tiles: the C read-modify-write dominates
-// and occupancy hides it (measured on MI355X at M = N = 4000..16000).
-template <> int default_cfg<double>(int ta, int tb, i64 m, i64 n, i64 k)
+// Default configuration by shape, from what the configurations measured
+// (table in tmvx_gemm_cfgs.h):
+//   - fewer 64 x 64 tiles than CUs: 32 x 32 tiles, four times as many (512^3
+//     FP64 26 -> 12 us; level with 64 x 64 at 1000^3, 256 tiles);
+//   - 128 x 128 tiles with at least four full turns over the 256 CUs and at
+//     most 3% of the last one idle, K deep enough that the traffic of C does
+//     not count: the fewest LDS reads per product (8192^3 FP64 15.3 ms against
+//     15.7; but 4.2 ms against 3.9 at 5000^3, 10% idle);
+//   - else 128 x 64 where C is large, 64 x 64 below and for a short K:
+//     several workgroups a CU hide each other's waits and the read and write
+//     of C (8192 x 8192 x 128 FP32 278-289 us against 302);
+//   - in FP32 a row-major B takes 128 x 64 in place of 128 x 128 tiles
+//     (4096^3: 1.05 ms against 1.22).
+template <typename T> int default_cfg(int tb, i64 m, i64 n, i64 k)
 {
-    if (m * n < 1024 * 1024) return (m * n <= 256 * 256) ? 4 : 0;
-    if (k <= 128) return 0;
-    return (!ta && !tb) ? 1 : 0;
-}
-template <> int default_cfg<float>(int ta, int tb, i64 m, i64 n, i64 k)
-{
-    if (m * n < 1024 * 1024 || k <= 128) return 3;
-    if (k <= 512) return 4;
-    if (!ta && !tb) return 0;
-    if (ta && !tb) return 2;
-    return 1;
+    constexpr bool D = sizeof(T) == 8;
+    constexpr int C64 = D ? 0 : 3, C128 = 1, C128x64 = 2, C32 = 4;
+    const i64 t64 = ((m + 63) / 64) * ((n + 63) / 64);
+    if (t64 < 256) return C32;
+    const i64 t128 = ((m + 127) / 128) * ((n + 127) / 128);
+    const i64 idle = (256 - t128 % 256) % 256;
+    if (t128 >= 1024 && k >= 1024 && 32 * idle <= t128) return !D && tb ? C128x64 : C128;
+    if (k <= 128) return C64;
+    return (double)m * (double)n >= (D ? 4.0e6 : 5.0e6) ? C128x64 : C64;
 }
 
 // Scale C by beta (k == 0 or alpha == 0): C = beta * C, or 0 when beta == 0.
@@ -84,7 +90,7 @@ int gemm_run(int cfg, int ta, int tb, i64 m, i64 n, i64 k, T alpha, const T* A,
         TMVX_CHECK_LAUNCH();
         return TMVX_OK;
     }
-    if (cfg < 0) cfg = default_cfg<T>(ta, tb, m, n, k);
+    if (cfg < 0) cfg = default_cfg<T>(tb, m, n, k);
     return GemmTable<T>::run(cfg, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, s);
 }
 
@@ -96,6 +102,23 @@ int gemm_launch(int ta, int tb, i64 m, i64 n, i64 k, T alpha, const T* A,
     return gemm_run<T>(-1, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, s);
 }
 
+// Large FP32 trailing updates beside a panel take 128 x 64 tiles of 32 deep
+// stages, one wave a SIMD: a panel's workgroups (two waves of 138 registers a
+// SIMD) must find room on a CU before the chain goes on, and a chip filled to
+// four waves a SIMD gives it late.  FP64 panels need a whole CU beside any
+// tile, so the faster tile wins.
+template <typename T>
+int gemm_launch_beside(int ta, int tb, i64 m, i64 n, i64 k, T alpha, const T* A, i64 lda,
+                       const T* B, i64 ldb, T beta, T* C, i64 ldc, hipStream_t s)
+{
+    const bool wide = sizeof(T) == 4 && k > 128 && (double)m * (double)n >= 1048576.0;
+    return gemm_run<T>(wide ? 6 : -1, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, s);
+}
+
+template int gemm_launch_beside<double>(int, int, i64, i64, i64, double, const double*, i64,
+                                        const double*, i64, double, double*, i64, hipStream_t);
+template int gemm_launch_beside<float>(int, int, i64, i64, i64, float, const float*, i64,
+                                       const float*, i64, float, float*, i64, hipStream_t);
 template int gemm_launch<double>(int, int, i64, i64, i64, double, const double*,
                                  i64, const double*, i64, double, double*, i64,
                                  hipStream_t);
@@ -109,74 +132,6 @@ static bool layouts_ok(int la, int lb)
            (lb == TMVX_COLMAJOR || lb == TMVX_ROWMAJOR);
 }
 
-// Row-major rows x cols (leading dimension ld) -> column-major copy with
-// leading dimension rows: 64 x 64 tiles through LDS, reads along the rows
-// and writes along the columns both coalesced.
-template <typename T>
-__global__ void __launch_bounds__(256)
-to_colmajor_kernel(i64 rows, i64 cols, const T* __restrict__ X, i64 ld, T* __restrict__ Y)
-{
-    __shared__ T tile[64][65];
-    const i64 r0 = (i64)blockIdx.y * 64, c0 = (i64)blockIdx.x * 64;
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;     // 64 x 4
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-        const int r = ty + 4 * q;
-        if (r0 + r < rows && c0 + tx < cols) tile[r][tx] = X[(r0 + r) * ld + c0 + tx];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-        const int c = ty + 4 * q;
-        if (c0 + c < cols && r0 + tx < rows) Y[(r0 + tx) + (c0 + c) * rows] = tile[tx][c];
-    }
-}
-
-template <typename T>
-static int to_colmajor(i64 rows, i64 cols, const T* X, i64 ld, T* Y, hipStream_t s)
-{
-    const i64 gy = (rows + 63) / 64, gx = (cols + 63) / 64;
-    if (gy > 65535 || gx > 0x7fffffff) return TMVX_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL(to_colmajor_kernel<T>, dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, s,
-                       rows, cols, X, ld, Y);
-    return hip_status(hipGetLastError());
-}
-
-// The public GEMM.  Large products with a row-major operand first copy that
-// operand to column-major (TMV likewise copies operands into its blocked
-// layout before its kernels, src/TMV_MultMM_Block.cpp:173-230): the
-// column-major MFMA kernel runs at 78% of the FP64 peak at 8192^3 against
-// 70% for the transposed-operand staging, and the copy costs one read and
-// one write of the operand.  The arithmetic, and so the result, is the same.
-template <typename T>
-int gemm_public(int la, int lb, i64 m, i64 n, i64 k, T alpha, const T* A, i64 lda,
-                const T* B, i64 ldb, T beta, T* C, i64 ldc, hipStream_t s)
-{
-    const bool big = (double)m * (double)n * (double)k >= 1073741824.0;   // 1024^3
-    if (!big || (la == TMVX_COLMAJOR && lb == TMVX_COLMAJOR) || alpha == T(0) || k == 0 ||
-        m <= 0 || n <= 0)
-        return gemm_run<T>(-1, la, lb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, s);
-    if (ldc < m || lda < (la ? k : m) || ldb < (lb ? n : k) || !A || !B || !C)
-        return TMVX_ERR_ARG;
-    const size_t na = la ? (size_t)m * (size_t)k : 0, nb = lb ? (size_t)k * (size_t)n : 0;
-    T* tmp = nullptr;
-    if (hipMallocAsync((void**)&tmp, sizeof(T) * (na + nb), s) != hipSuccess) {
-        (void)hipGetLastError();           // no room for the copy: stage in place
-        return gemm_run<T>(-1, la, lb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, s);
-    }
-    int rc = TMVX_OK;
-    const T* Ac = A;
-    const T* Bc = B;
-    i64 ldac = lda, ldbc = ldb;
-    if (la) { rc = to_colmajor<T>(m, k, A, lda, tmp, s); Ac = tmp; ldac = m; }
-    if (rc == TMVX_OK && lb) { rc = to_colmajor<T>(k, n, B, ldb, tmp + na, s); Bc = tmp + na; ldbc = k; }
-    if (rc == TMVX_OK)
-        rc = gemm_run<T>(-1, TMVX_COLMAJOR, TMVX_COLMAJOR, m, n, k, alpha, Ac, ldac, Bc, ldbc,
-                         beta, C, ldc, s);
-    (void)hipFreeAsync(tmp, s);
-    return rc;
-}
-
 } // namespace tmvx
 
 extern "C" {
@@ -186,7 +141,7 @@ int tmvx_gemm_f64(int la, int lb, int64_t m, int64_t n, int64_t k, double alpha,
                   double beta, double* C, int64_t ldc, void* stream)
 {
     if (!tmvx::layouts_ok(la, lb)) return TMVX_ERR_ARG;
-    return tmvx::gemm_public<double>(la, lb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc,
+    return tmvx::gemm_launch<double>(la, lb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc,
                                      (hipStream_t)stream);
 }
 
@@ -195,7 +150,7 @@ int tmvx_gemm_f32(int la, int lb, int64_t m, int64_t n, int64_t k, float alpha,
                   float beta, float* C, int64_t ldc, void* stream)
 {
     if (!tmvx::layouts_ok(la, lb)) return TMVX_ERR_ARG;
-    return tmvx::gemm_public<float>(la, lb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc,
+    return tmvx::gemm_launch<float>(la, lb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc,
                                     (hipStream_t)stream);
 }
 

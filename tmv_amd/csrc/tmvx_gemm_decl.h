@@ -17,6 +17,9 @@ struct GemmCfg {
     static constexpr int PADX = 16 / sizeof(T);      // pad of k-major rows (16 B)
     static constexpr int NVA = BM * BK / V / NT;     // 16 B loads per thread
     static constexpr int NVB = BN * BK / V / NT;
+    // stages in flight: two where several workgroups a CU also cover the
+    // loads, four where a workgroup has the CU (nearly) to itself
+    static constexpr int P = NVA + NVB <= 4 && MINW < 4 ? 4 : 2;
     static_assert(BM % (16 * WM) == 0 && BN % (16 * WN) == 0, "wave tile");
     static_assert(BK % 16 == 0, "BK must be a multiple of 16");
     static_assert((BM * BK) % (V * NT) == 0 && (BN * BK) % (V * NT) == 0, "loads");

@@ -86,8 +86,8 @@ gemm_kernel(i64 M, i64 N, i64 K, T alpha, const T* __restrict__ A, i64 lda,
 #pragma unroll
         for (int j = 0; j < Cfg::FN; ++j) acc[i][j] = Acc{0, 0, 0, 0};
 
-    VT ra[Cfg::NVA], rb[Cfg::NVB];
-    const bool full_mn = (m0 + BM <= M) && (n0 + BN <= N);
+    constexpr int P = Cfg::P;
+    VT ra[P][Cfg::NVA], rb[P][Cfg::NVB];
 
     // Thread -> (row x, k) of its v-th 16-byte vector.  The vector runs
     // along k when the operand is k-contiguous, else along x.
@@ -98,51 +98,75 @@ gemm_kernel(i64 M, i64 N, i64 K, T alpha, const T* __restrict__ A, i64 lda,
 
     // ---- global -> registers -------------------------------------------
     // 16-byte loads need element alignment only (global_load_dwordx4 takes
-    // any dword address), so an odd leading dimension or base takes them too;
-    // a vector that crosses the edge of the matrix is read by element.
+    // any dword address), so odd leading dimensions and bases take them too.
+    // Rows past the edge of the matrix are clamped to its last row or vector:
+    // what they hold only reaches entries of C that are not stored, and no
+    // branch stands between a stage's loads and those of the next (the wait
+    // for one stage must not wait for the ones issued after it).
+    //   pa, pb: source of the thread's r-th vector in the next stage to load;
+    //   ea, eb: the last entry of that vector inside the matrix, where the
+    //   vector runs along the rows and the edge splits it (RAG).
     typedef VT VU __attribute__((aligned(sizeof(T))));
-    auto load_op = [&](const T* X, i64 ld, bool kc, i64 x0, i64 xn, i64 k0, bool fast, int rows,
-                       auto nv, VT* rx) __attribute__((always_inline)) {
+    const T* pa[Cfg::NVA];
+    const T* pb[Cfg::NVB];
+    int ea[Cfg::NVA], eb[Cfg::NVB];
+    auto source = [&](const T* X, i64 ld, bool kc, i64 x0, i64 xn, int rows, auto nv, const T** p,
+                      int* le) __attribute__((always_inline)) {
 #pragma unroll
         for (int r = 0; r < decltype(nv)::value; ++r) {
             int x, k;
             vcoord(t + r * NT, rows, kc, x, k);
-            const i64 gx = x0 + x, gk = k0 + k;
-            const T* p = kc ? X + gx * ld + gk : X + gx + gk * ld;
-            if (fast) {
-                rx[r] = *reinterpret_cast<const VU*>(p);
-            } else {
-                const i64 nx = xn - gx, nkk = K - gk;       // entries left along x and k
-                const i64 along = kc ? nkk : nx, across = kc ? nx : nkk;
-                if (across > 0 && along >= V) {
-                    rx[r] = *reinterpret_cast<const VU*>(p);
-                } else {
-#pragma unroll
-                    for (int e = 0; e < V; ++e)
-                        rx[r][e] = (across > 0 && e < along) ? p[e] : T(0);
-                }
-            }
+            i64 gx = x0 + x;
+            // (the edge splits no vector: its last whole one; otherwise by entry)
+            const i64 gmax = (kc || xn % V) ? xn - 1 : xn - V;
+            gx = gx < gmax ? gx : gmax;
+            le[r] = xn - 1 - gx < V - 1 ? (int)(xn - 1 - gx) : V - 1;
+            p[r] = kc ? X + gx * ld + k : X + gx + (i64)k * ld;
         }
     };
-    auto load = [&](i64 k0) __attribute__((always_inline)) {
-        const bool fast = full_mn && (k0 + BK <= K);
-        load_op(A, lda, AKC, m0, M, k0, fast, BM, std::integral_constant<int, Cfg::NVA>(), ra);
-        load_op(B, ldb, BKC, n0, N, k0, fast, BN, std::integral_constant<int, Cfg::NVB>(), rb);
+    source(A, lda, AKC, m0, M, BM, std::integral_constant<int, Cfg::NVA>(), pa, ea);
+    source(B, ldb, BKC, n0, N, BN, std::integral_constant<int, Cfg::NVB>(), pb, eb);
+    const i64 stepa = AKC ? BK : BK * lda, stepb = BKC ? BK : BK * ldb;
+    auto load_full = [&](VT* rx, const T** p, const int* le, bool split, i64 step, auto nv)
+        __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < decltype(nv)::value; ++r) {
+            if (split) {
+#pragma unroll
+                for (int e = 0; e < V; ++e) rx[r][e] = p[r][e < le[r] ? e : le[r]];
+            } else {
+                rx[r] = *reinterpret_cast<const VU*>(p[r]);
+            }
+            p[r] += step;
+        }
+    };
+    // the last stage when BK does not divide K: entries past K are zero
+    auto load_tail = [&](VT* rx, const T** p, const int* le, bool kc, i64 ld, i64 k0, int rows, auto nv)
+        __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < decltype(nv)::value; ++r) {
+            int x, k;
+            vcoord(t + r * NT, rows, kc, x, k);
+            const i64 left = K - k0 - k;
+#pragma unroll
+            for (int e = 0; e < V; ++e)
+                rx[r][e] = (kc ? e < left : left > 0) ? p[r][kc ? e : e < le[r] ? e : le[r]] : T(0);
+        }
     };
 
     // ---- registers -> LDS (same orientation, one 16-byte store each) ----
-    auto store = [&](int buf) {
+    auto store = [&](int buf, const VT* xa, const VT* xb) __attribute__((always_inline)) {
 #pragma unroll
         for (int r = 0; r < Cfg::NVA; ++r) {
             int x, k;
             vcoord(t + r * NT, BM, AKC, x, k);
-            *reinterpret_cast<VT*>(&As[buf][SA::idx(x, k)]) = ra[r];
+            *reinterpret_cast<VT*>(&As[buf][SA::idx(x, k)]) = xa[r];
         }
 #pragma unroll
         for (int r = 0; r < Cfg::NVB; ++r) {
             int x, k;
             vcoord(t + r * NT, BN, BKC, x, k);
-            *reinterpret_cast<VT*>(&Bs[buf][SB::idx(x, k)]) = rb[r];
+            *reinterpret_cast<VT*>(&Bs[buf][SB::idx(x, k)]) = xb[r];
         }
     };
 
@@ -159,7 +183,7 @@ gemm_kernel(i64 M, i64 N, i64 K, T alpha, const T* __restrict__ A, i64 lda,
             for (int s = 0; s < 4; ++s) f[s] = S[(kb + 4 * g + s) * ld + x];
         }
     };
-    auto compute = [&](int buf) {
+    auto compute = [&](int buf) __attribute__((always_inline)) {
         const int am = wm * Cfg::TM + r16;
         const int bn = wn * Cfg::TN + r16;
 #pragma unroll
@@ -179,18 +203,61 @@ gemm_kernel(i64 M, i64 N, i64 K, T alpha, const T* __restrict__ A, i64 lda,
         }
     };
 
-    const i64 nk = (K + BK - 1) / BK;
-    if (nk > 0) {
-        load(0);
-        store(0);
+    // ---- P stages in flight --------------------------------------------
+    // One stage in flight left every step of a tile waiting a load's latency
+    // (1000^3 FP64, one workgroup a CU: 110 us; with P stages 47 us).
+    // Stage s is loaded into register set s mod P while stages s - P .. s - 1
+    // are worked on, and goes to LDS buffer s mod 2 one step ahead.
+    const i64 nk = (K + BK - 1) / BK, nfull = K / BK;
+    auto run = [&](auto rag) __attribute__((always_inline)) {
+        constexpr bool RA = decltype(rag)::value && !AKC, RB = decltype(rag)::value && !BKC;
+        constexpr std::integral_constant<int, Cfg::NVA> nva{};
+        constexpr std::integral_constant<int, Cfg::NVB> nvb{};
+        auto load = [&](VT* xa, VT* xb) __attribute__((always_inline)) {
+            load_full(xa, pa, ea, RA, stepa, nva);
+            load_full(xb, pb, eb, RB, stepb, nvb);
+        };
+        auto load_any = [&](i64 st, VT* xa, VT* xb) __attribute__((always_inline)) {
+            if (st < nfull) {
+                load(xa, xb);
+            } else if (st < nk) {
+                load_tail(xa, pa, ea, AKC, lda, st * BK, BM, nva);
+                load_tail(xb, pb, eb, BKC, ldb, st * BK, BN, nvb);
+            }
+        };
+        static_for<0, P>([&](auto sc) __attribute__((always_inline)) {
+            constexpr int q = decltype(sc)::value;
+            load_any(q, ra[q], rb[q]);
+        });
+        store(0, ra[0], rb[0]);
+        load_any(P, ra[0], rb[0]);
         __syncthreads();
-        for (i64 kt = 0; kt < nk; ++kt) {
-            const int buf = (int)(kt & 1);
-            if (kt + 1 < nk) load((kt + 1) * BK);
-            compute(buf);
-            if (kt + 1 < nk) store(buf ^ 1);
-            __syncthreads();
-        }
+        i64 kt = 0;
+        for (; kt + 2 * P < nfull; kt += P)
+            static_for<0, P>([&](auto uc) __attribute__((always_inline)) {
+                constexpr int u = decltype(uc)::value, q = (u + 1) % P;
+                store((u + 1) & 1, ra[q], rb[q]);
+                load(ra[q], rb[q]);
+                compute(u & 1);
+                __syncthreads();
+            });
+        for (; kt < nk; kt += P)
+            static_for<0, P>([&](auto uc) __attribute__((always_inline)) {
+                constexpr int u = decltype(uc)::value, q = (u + 1) % P;
+                if (kt + u >= nk) return;
+                if (kt + u + 1 < nk) {
+                    store((u + 1) & 1, ra[q], rb[q]);
+                    load_any(kt + u + 1 + P, ra[q], rb[q]);
+                }
+                compute(u & 1);
+                __syncthreads();
+            });
+    };
+    // the edge splits a vector that runs along the rows
+    const bool split = (!AKC && m0 + BM > M && M % V) || (!BKC && n0 + BN > N && N % V);
+    if (nk > 0) {
+        if (split) run(std::true_type());
+        else run(std::false_type());
     }
 
     // ---- epilogue: acc[i][j][r] = C[row(g, r)][r16] of block (i, j) -----

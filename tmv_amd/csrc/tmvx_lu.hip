@@ -1146,7 +1146,8 @@ int getrf_nb_impl(i64 m, i64 n, T* A, i64 lda, i64* piv, i64* perm, i64* info, h
                 return gemm_lowp_launch(lowprec, rows, cols, K, -1.0f, A21, lda, U12, lda, 1.0f,
                                         A22, lda, word, st);
         }
-        return gemm_launch<T>(0, 0, rows, cols, K, T(-1), A21, lda, U12, lda, T(1), A22, lda, st);
+        const auto go = st == s ? gemm_launch<T> : gemm_launch_beside<T>;
+        return go(0, 0, rows, cols, K, T(-1), A21, lda, U12, lda, T(1), A22, lda, st);
     };
 
     int rc = TMVX_OK;
