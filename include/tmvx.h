@@ -162,8 +162,7 @@ int tmvx_gemm_c(int layout_a, int layout_b, int conj_a, int conj_b, int64_t m, i
  * elements).  The pivot is the candidate of largest modulus, first row on
  * ties; a column whose largest candidate underflows is zeroed from the
  * diagonal down with piv[j] = j, and *info (host) gets the 1-based first
- * zero pivot, or 0.  Synchronises.  The complex path is functional, not
- * tuned: one workgroup per panel, trailing updates on the complex GEMM.
+ * zero pivot, or 0.  Synchronises.  One workgroup per panel.
  * Replaces: tmv::LU_Decompose for complex T (src/TMV_LUDecompose.cpp:217-407,
  * 443-462).
  */
@@ -205,7 +204,7 @@ int tmvx_getri_z(int64_t n, const double* LU, int64_t lda, const int64_t* piv, d
  * it (first elements 1, implicit); beta (device, n) the reflectors' scales,
  * H_j = I - beta_j v_j v_j^T, A = H_0 H_1 ... H_{n-1} R.  Reflectors as
  * TMV's HouseholderReflect builds them (R(j,j) = -sign(x0) |x|, zero or
- * underflowing columns give beta = 0).  Functional, not tuned.
+ * underflowing columns give beta = 0).
  * Replaces: tmv::QR_Decompose(MatrixView A, VectorView beta, T& det)
  * (src/TMV_QRDecompose.cpp:603-650; reflector src/TMV_Householder.cpp:46-180).
  */
