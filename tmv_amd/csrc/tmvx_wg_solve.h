@@ -9,12 +9,17 @@
 // 369-410).  Entries are divided by U's diagonal, a zero entry stays zero
 // (src/TMV_TriDiv_V.cpp:187).
 //
-// The triangle is walked in blocks of 16 rows.  The right-hand sides still
-// to be solved are MFMA accumulators (16 rows x 16 right-hand sides each,
-// the 16-row blocks dealt out to the waves); a solved block's product with
-// the rows to come is one 16x16x16 MFMA step per block row, with the factor
-// entries loaded a block ahead.  The diagonal block itself is a plain
-// substitution, a right-hand side per lane, its entries broadcast from LDS.
+// The triangle is walked in blocks of 16 rows.  The sums of products that the
+// rows to come will take off their right-hand sides are MFMA accumulators (16
+// rows x 16 right-hand sides each, the 16-row blocks dealt out to the waves);
+// a solved block's product with the rows to come is one 16x16x16 MFMA step per
+// block row, with the factor entries loaded a block ahead.  The diagonal block
+// itself is a plain substitution, a right-hand side per lane, its entries
+// broadcast from LDS.  A row's products are summed apart from its right-hand
+// side and subtracted once: taken off one after another, each would be rounded
+// at the size of the right-hand side (A^T X = B, n = 256, A uniform + n I:
+// error 3.4 eps so, 0.36 eps apart, as the wave form's dot products), and each
+// block's sum is formed by itself before it joins that of the blocks before.
 // One barrier per block: the chain is 16 substitution steps per block
 // instead of a wave-wide sweep (or a wave sum, for A^T) per row, and four
 // waves stream the factors of one system.
@@ -24,11 +29,14 @@
 namespace tmvx {
 
 // Batches of up to this many systems take the workgroup form; larger ones
-// fill the GPU with a wave per system (tmvx_wave_solve.h), which keeps
-// eight systems in flight where this form, by its LDS, keeps two: measured
-// FP64 with one right-hand side, 512 systems of n = 256 314 -> 143 us
-// (transposed 286 -> 136), n = 200 135 -> 94 us, 300 of n = 64 42 -> 28 us,
-// but 2000 of n = 128 97 -> 224 us and 4000 of n = 65 91 -> 234 us.
+// fill the GPU with a wave per system (tmvx_wave_solve.h), which keeps eight
+// systems in flight where this form, by its LDS and registers, keeps two.
+// Wave form -> workgroup form, FP64, transposed, one right-hand side (us):
+//   512 systems:  n = 64 72 -> 42, n = 128 137 -> 63, n = 256 274 -> 145
+//   640:          n = 64 73 -> 42, n = 128 138 -> 101, n = 256 278 -> 265
+//   1024:         n = 64 73 -> 43, n = 128 138 -> 114, n = 200 220 -> 208,
+//                 n = 256 281 -> 295 (four right-hand sides 1081 -> 301)
+// and, untransposed, 2000 of n = 128 97 -> 224, 4000 of n = 65 91 -> 234.
 constexpr int WS_WG_MAX = 1024;
 
 constexpr int WS_RHS = 16;                 // right-hand sides per pass
@@ -54,6 +62,7 @@ struct WgSolveLds {
     static constexpr int NMAX = 16 * WS_TPW * NWV;
     T x[NMAX][WS_RHS];
     T d[NMAX / 16][16][16];                // d[b][k][i] = op(A)(16 b + i, 16 b + k)
+    T s[16][WS_RHS];                       // the next block's sums of products
     short src[NMAX];                       // row i of P A is row src[i] of A
     short piv[NMAX];
 };
@@ -73,6 +82,7 @@ __device__ __forceinline__ void wg_trsv(int n, const T* __restrict__ A, int ld,
         L.d[b][k & 15][i & 15] = (i < n && k < n) ? (TRANS ? A[k + i * ld] : A[i + k * ld])
                                                   : (i == k ? T(1) : T(0));
     }
+    for (int e = tid; e < 16 * WS_RHS; e += 64 * NWV) L.s[e / WS_RHS][e % WS_RHS] = T(0);
     // op(A)(16 tb + li, 16 b + k(s, g)), the MFMA k slot (s, g) holding
     // k = 4 s + g, or 4 g + s where k is the contiguous index of A
     auto frag = [&](int tb, int b, T (&f)[4]) __attribute__((always_inline)) {
@@ -95,25 +105,24 @@ __device__ __forceinline__ void wg_trsv(int n, const T* __restrict__ A, int ld,
         const int tb = wave + NWV * t;
         static_for<0, 4>([&](auto rc) __attribute__((always_inline)) {
             constexpr int r = decltype(rc)::value;
-            acc[t][r] = L.x[16 * tb + Mfma<T>::row(g, r)][li];
+            acc[t][r] = T(0);
         });
         if (later(tb, first)) frag(tb, first, f[t]);
     });
-    sync();                                   // L.d complete
+    sync();                                   // L.d and L.s complete
     for (int q = 0; q < nb; ++q) {
         const int b = LOWER ? q : nb - 1 - q, bn = LOWER ? b + 1 : b - 1;
         if (NWV == 1 || wave == b % NWV) {
-            // the block's right-hand sides through LDS to one per lane
-            // (every lane group solves the same 16)
+            // the block through LDS to one right-hand side per lane (every lane
+            // group solves the same 16); x[k] is the sum of the block's own
+            // products of row k, then its solution
             T x[16];
-            static_for<0, 16>([&](auto kc) __attribute__((always_inline)) {
-                constexpr int k = decltype(kc)::value;
-                x[k] = L.x[16 * b + k][li];
-            });
-            // column k of the diagonal block is read one step before its use
-            // (the offset passes through an empty asm statement with the
-            // previous entry, or all 120 reads would be hoisted to the top)
-            T d[16];
+            static_for<0, 16>([&](auto kc) __attribute__((always_inline)) { x[decltype(kc)::value] = T(0); });
+            // column k of the diagonal block, row k's right-hand side and its
+            // sum so far are read one step before their use (the offset passes
+            // through an empty asm statement with the previous entry, or all
+            // the reads would be hoisted to the top)
+            T d[16], bk = L.x[16 * b + (LOWER ? 0 : 15)][li], sk = L.s[LOWER ? 0 : 15][li];
             int off = 0;
             auto dcol = [&](auto kc, T (&c)[16]) __attribute__((always_inline)) {
                 constexpr int k = decltype(kc)::value;
@@ -125,15 +134,22 @@ __device__ __forceinline__ void wg_trsv(int n, const T* __restrict__ A, int ld,
             dcol(std::integral_constant<int, LOWER ? 0 : 15>{}, d);
             static_for<0, 16>([&](auto qc) __attribute__((always_inline)) {
                 constexpr int q = decltype(qc)::value, k = LOWER ? q : 15 - q;
-                T dn[16];
+                T dn[16], bn = T(0), sn = T(0);
                 if constexpr (q > 0) __asm__ volatile("" : "+v"(off) : "v"(x[k]));
-                if constexpr (q < 15) dcol(std::integral_constant<int, LOWER ? k + 1 : k - 1>{}, dn);
+                if constexpr (q < 15) {
+                    dcol(std::integral_constant<int, LOWER ? k + 1 : k - 1>{}, dn);
+                    bn = (&L.x[16 * b + (LOWER ? k + 1 : k - 1)][li])[off];
+                    sn = (&L.s[LOWER ? k + 1 : k - 1][li])[off];
+                }
+                x[k] = bk - (sk + x[k]);
                 if constexpr (!UNIT) x[k] = x[k] == T(0) ? T(0) : x[k] / d[k];
                 static_for<0, 16>([&](auto ic) __attribute__((always_inline)) {
                     constexpr int i = decltype(ic)::value;
-                    if constexpr (LOWER ? i > k : i < k) x[i] -= d[i] * x[k];
+                    if constexpr (LOWER ? i > k : i < k) x[i] = fma(d[i], x[k], x[i]);
                     if constexpr (q < 15) d[i] = dn[i];
                 });
+                bk = bn;
+                sk = sn;
             });
             if (g == 0)
                 static_for<0, 16>([&](auto kc) __attribute__((always_inline)) {
@@ -154,14 +170,16 @@ __device__ __forceinline__ void wg_trsv(int n, const T* __restrict__ A, int ld,
                 constexpr int t = decltype(tc)::value;
                 const int tb = wave + NWV * t;
                 if ((tb == bn) != (decltype(pc)::value == 0) || !later(tb, b)) return;   // uniform
+                v4 p = {T(0), T(0), T(0), T(0)};
                 static_for<0, 4>([&](auto sc) __attribute__((always_inline)) {
                     constexpr int s = decltype(sc)::value;
-                    acc[t] = Mfma<T>::mac(-f[t][s], xb[s], acc[t]);
+                    p = Mfma<T>::mac(f[t][s], xb[s], p);
                 });
+                acc[t] += p;
                 if constexpr (decltype(pc)::value == 0)
                     static_for<0, 4>([&](auto rc) __attribute__((always_inline)) {
                         constexpr int r = decltype(rc)::value;
-                        L.x[16 * tb + Mfma<T>::row(g, r)][li] = acc[t][r];
+                        L.s[Mfma<T>::row(g, r)][li] = acc[t][r];
                     });
             });
         });
@@ -170,7 +188,7 @@ __device__ __forceinline__ void wg_trsv(int n, const T* __restrict__ A, int ld,
             const int tb = wave + NWV * t;
             if (later(tb, bn)) frag(tb, bn, f[t]);       // in flight during the next block
         });
-        WaveSync()();                         // the owner's block is in LDS for its own reads
+        WaveSync()();                         // the owner's sums are in LDS for its own reads
     }
 }
 
