@@ -154,7 +154,9 @@ __device__ __forceinline__ void wg_trsv(int n, const T* __restrict__ A, int ld,
             if (g == 0)
                 static_for<0, 16>([&](auto kc) __attribute__((always_inline)) {
                     constexpr int k = decltype(kc)::value;
-                    L.x[16 * b + k][li] = x[k];
+                    // (rows past n stay zero: the next sweep starts from them, and
+                    // an Inf or NaN there would reach every row)
+                    L.x[16 * b + k][li] = 16 * b + k < n ? x[k] : T(0);
                 });
         }
         sync();
