@@ -65,6 +65,7 @@ struct WgSolveLds {
     T s[16][WS_RHS];                       // the next block's sums of products
     short src[NMAX];                       // row i of P A is row src[i] of A
     short piv[NMAX];
+    int bad;                               // right-hand sides whose solution holds a NaN
 };
 
 // One triangular solve on L.x (rows past n are zero), A with leading
@@ -194,6 +195,32 @@ __device__ __forceinline__ void wg_trsv(int n, const T* __restrict__ A, int ld,
     }
 }
 
+// Column c of L.x := U^-1 L^-1 P b by one wave, a column of LU at a time.
+template <typename T, int NWV>
+__device__ __forceinline__ void plain_getrs(int n, const T* __restrict__ LU, const T* b,
+                                            WgSolveLds<T, NWV>& L, int c, int lane)
+{
+#pragma clang loop unroll(disable)
+    for (int i = lane; i < n; i += 64) L.x[i][c] = b[(int)L.src[i]];
+    WaveSync()();
+#pragma clang loop unroll(disable)
+    for (int q = 0; q < 2 * n; ++q) {
+        const bool low = q < n;                    // L forward, then U backward
+        const int k = low ? q : 2 * n - 1 - q;
+        T x = L.x[k][c];
+        if (!low && x != T(0)) {
+            x = x / LU[k + k * n];
+            L.x[k][c] = x;
+        }
+        if (x != T(0)) {
+#pragma clang loop unroll(disable)
+            for (int i = low ? k + 1 + lane : lane; i < (low ? n : k); i += 64)
+                L.x[i][c] -= LU[i + k * n] * x;
+        }
+        WaveSync()();
+    }
+}
+
 // X := A^-1 B (A^-T B) for nr right-hand sides, B and X n x nr with leading
 // dimension n (X may be B).
 template <typename T, int NWV, bool TRANS, class Sync>
@@ -226,10 +253,26 @@ __device__ __forceinline__ void wg_getrs(int n, int nr, const T* __restrict__ LU
             if (i < n && c < nc) v = B[(TRANS ? i : (int)L.src[i]) + (i64)(c0 + c) * n];
             L.x[i][c] = v;
         }
+        if (tid == 0) L.bad = 0;
         sync();
         if constexpr (!TRANS) {
             wg_trsv<T, NWV, false, true, true>(n, LU, n, L, tid, sync);
             wg_trsv<T, NWV, false, false, false>(n, LU, n, L, tid, sync);
+            // A NaN may come from a product that the substitution leaves out (a
+            // zero entry takes no part in it, src/TMV_TriDiv_V.cpp:187, but a
+            // zero times an Inf of the factors does in a matrix step): such
+            // columns are solved again by plain column sweeps, a wave each.
+            for (int e = tid; e < nc * n; e += NT) {
+                const T v = L.x[e % n][e / n];
+                if (v != v) atomicOr(&L.bad, 1 << (e / n));
+            }
+            sync();
+            const int bad = __builtin_amdgcn_readfirstlane(L.bad);
+            if (bad) {
+                for (int c = NWV == 1 ? 0 : tid >> 6; c < nc; c += NWV)
+                    if ((bad >> c) & 1) plain_getrs<T, NWV>(n, LU, B + (i64)(c0 + c) * n, L, c, tid & 63);
+                sync();
+            }
         } else {
             wg_trsv<T, NWV, true, true, false>(n, LU, n, L, tid, sync);
             wg_trsv<T, NWV, true, false, true>(n, LU, n, L, tid, sync);
