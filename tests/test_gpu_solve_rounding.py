@@ -92,3 +92,32 @@ def test_batched_transposed_solve(dev, dtype, n):
     tmv_amd.gesv_adjoint_batched(b, w, w, grad, grad)
     x = np.stack([grad.b(i).cpu().numpy() for i in range(cnt)])
     assert rms_error(x, ref) <= 0.75 * eps
+
+
+def factor(A, P):
+    """Packed LU of A with given interchanges, in long double."""
+    A, n = wide(A).copy(), len(P)
+    for k, p in enumerate(P):
+        if p != k:
+            A[[k, int(p)]] = A[[int(p), k]]
+        A[k + 1:, k] /= A[k, k]
+        A[k + 1:, k + 1:] -= np.outer(A[k + 1:, k], A[k, k + 1:])
+    return A
+
+
+@pytest.mark.parametrize("dtype", [torch.complex128, torch.complex64])
+@pytest.mark.parametrize("n", [200, 400])
+def test_complex_lu(dev, dtype, n):
+    """Complex factors.  An entry takes a rounding at its size for each panel
+    of 16 columns before it (25 at n = 400), the rest of its products being
+    summed first, and one for each column of its own panel before it (7 on
+    average); eps / 2 / sqrt(3) rms each, of the entries that carry most of the
+    norm (the diagonal, whose size hides half of that): bar 1.5 eps."""
+    npt = np.complex128 if dtype == torch.complex128 else np.complex64
+    eps = EPS64 if dtype == torch.complex128 else EPS32
+    A = matrix(np.random.default_rng(n), n, cplx=True).astype(npt)
+    print(f"getrf_complex n {n} {dtype}", flush=True)
+    a = tmv_amd.colmajor(torch.from_numpy(A).cuda())
+    piv, info = tmv_amd.getrf_complex(a)
+    assert info == 0
+    assert rms_error(a.cpu().numpy(), factor(A, piv.cpu().numpy())) <= 1.5 * eps

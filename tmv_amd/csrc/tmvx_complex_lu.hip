@@ -184,12 +184,15 @@ constexpr int ZN_NTH = 512;              // panel workgroup
 constexpr int ZN_NW = ZN_NTH / 64;
 constexpr i64 ZN_MMAX = 4 * ZN_NTH;      // rows a panel can hold (four a thread)
 
-// x -= l u
-template <typename Z> __device__ __forceinline__ void csubmul(Z& x, Z l, Z u)
+// s += l u
+template <typename Z> __device__ __forceinline__ void caddmul(Z& s, Z l, Z u)
 {
-    x.x = fma(-l.x, u.x, fma(l.y, u.y, x.x));
-    x.y = fma(-l.x, u.y, fma(-l.y, u.x, x.y));
+    s.x = fma(l.x, u.x, fma(-l.y, u.y, s.x));
+    s.y = fma(l.x, u.y, fma(l.y, u.x, s.y));
 }
+// x -= l u: the product first, or x would take two roundings at its size
+template <typename Z> __device__ __forceinline__ void csubmul(Z& x, Z l, Z u)
+{ x = csub(x, cmul(l, u)); }
 template <int C, typename Z> __device__ __forceinline__ Z row_bcast_z(Z v)
 {
     Z r;
@@ -198,7 +201,7 @@ template <int C, typename Z> __device__ __forceinline__ Z row_bcast_z(Z v)
     return r;
 }
 
-// x -= sum over k in [K0, K0 + 4) of l[k] (lane k of each row of 16 lanes of u),
+// (xr, xi) -= sum over k in [K0, K0 + 4) of l[k] (lane k of each row of 16 lanes of u),
 // given -u.x, -u.y and u.y: broadcast and multiply-add in one instruction
 // (cf. bcast_fma8).  Call with every lane active.
 #define ZN_STEP(SUF, K, LX, LY)                                                              \
@@ -371,8 +374,8 @@ znupdate_kernel(i64 n, typename CplxT<R>::type* __restrict__ Ag, i64 lda, i64 j0
         // column 4 wave + g, row li
         const int c = 4 * wave + g;
         const bool in = c < nc && li < NB;
-        Z x, l[NB];
-        x.x = x.y = R(0);
+        Z x, sum, l[NB];                     // (products summed apart from x)
+        x.x = x.y = sum.x = sum.y = R(0);
         if (in) x = A[from[li] + (c0 + c) * lda];
 #pragma unroll
         for (int k = 0; k < NB; ++k) {
@@ -381,10 +384,10 @@ znupdate_kernel(i64 n, typename CplxT<R>::type* __restrict__ Ag, i64 lda, i64 j0
         }
         static_for<0, NB>([&](auto kc) __attribute__((always_inline)) {
             constexpr int k = decltype(kc)::value;
-            const Z xk = row_bcast_z<k>(x);
-            if (li > k) csubmul(x, l[k], xk);
+            const Z xk = row_bcast_z<k>(csub(x, sum));
+            if (li > k) caddmul(sum, l[k], xk);
         });
-        s_u[c][li] = x;
+        s_u[c][li] = csub(x, sum);
     }
     __syncthreads();
     for (int r0 = NB + 64 * wave; r0 < m; r0 += 256) {
@@ -398,9 +401,12 @@ znupdate_kernel(i64 n, typename CplxT<R>::type* __restrict__ Ag, i64 lda, i64 j0
         for (int c = 0; c < ZU_CW; ++c) {
             const Z uv = s_u[c][li];
             const R nux = -uv.x, nuy = -uv.y;
+            R sr = R(0), si = R(0);          // minus the products, summed apart from x
             static_for<0, NB / 4>([&](auto kc) __attribute__((always_inline)) {
-                zbcast_fma4<4 * decltype(kc)::value>(x[c].x, x[c].y, nux, nuy, uv.y, l);
+                zbcast_fma4<4 * decltype(kc)::value>(sr, si, nux, nuy, uv.y, l);
             });
+            x[c].x += sr;
+            x[c].y += si;
         }
         if (r < m) {
 #pragma unroll
