@@ -121,3 +121,23 @@ def test_complex_lu(dev, dtype, n):
     piv, info = tmv_amd.getrf_complex(a)
     assert info == 0
     assert rms_error(a.cpu().numpy(), factor(A, piv.cpu().numpy())) <= 1.5 * eps
+
+
+@pytest.mark.parametrize("dtype", [torch.complex128, torch.complex64])
+@pytest.mark.parametrize("trans", [False, True])
+def test_complex_solve(dev, dtype, trans):
+    """Complex solves with given factors.  A sweep goes over an entry once for
+    each block of 16 rows before it and sums the products of its own block, so
+    an entry of the first sweep takes n / 16 roundings at most and n / 32 on
+    average, the second as many: 25 at n = 400, of eps / 2 / sqrt(3) rms a
+    component or 1.5 eps; the quotients' own 2 eps beside: bar 3 eps."""
+    npt = np.complex128 if dtype == torch.complex128 else np.complex64
+    eps = EPS64 if dtype == torch.complex128 else EPS32
+    n, g = 400, np.random.default_rng(7)
+    LU, P = host_lu(matrix(g, n, cplx=True).astype(npt))
+    B = (g.standard_normal((n, 3)) + 1j * g.standard_normal((n, 3))).astype(npt)
+    print(f"getrs_complex trans {trans} {dtype}", flush=True)
+    lu = tmv_amd.colmajor(torch.from_numpy(LU).cuda())
+    x = tmv_amd.colmajor(torch.from_numpy(B).cuda())
+    tmv_amd.getrs_complex(lu, torch.from_numpy(P).cuda(), x, trans=trans)
+    assert rms_error(x.cpu().numpy(), solve(LU, P, B, trans)) <= 3 * eps

@@ -663,7 +663,11 @@ __device__ __forceinline__ void zsolve_sweep(int n, const typename CplxT<R>::typ
         load(r0 + t < r1 ? r0 + t : -1, b, a);
         if (t < 64) {
             const int r = 16 * b + li;
-            Z x = r < n ? s_b[r] : zero, d[16], dd = zero;
+            // x: the entry less its products so far, formed anew in each step from
+            // b less the sum of all but the last product (one fewer operation
+            // on the chain than b less the whole sum)
+            const Z bv = r < n ? s_b[r] : zero;
+            Z x = bv, sum = zero, d[16], dd = zero;
             load(r, b, d);
             if constexpr (diag) {
                 static_for<0, 16>([&](auto kc) __attribute__((always_inline)) {
@@ -685,7 +689,12 @@ __device__ __forceinline__ void zsolve_sweep(int n, const typename CplxT<R>::typ
                     }
                 }
                 const Z xk = row_bcast_z<k>(x);
-                if (fwd ? li > k : li < k) csubmul(x, d[k], xk);
+                if (fwd ? li > k : li < k) {
+                    const Z bs = csub(bv, sum);
+                    x.x = fma(-d[k].x, xk.x, fma(d[k].y, xk.y, bs.x));
+                    x.y = fma(-d[k].x, xk.y, fma(-d[k].y, xk.x, bs.y));
+                    caddmul(sum, d[k], xk);
+                }
             });
             if (lane < 16 && r < n) s_b[r] = x;
         }
@@ -695,10 +704,12 @@ __device__ __forceinline__ void zsolve_sweep(int n, const typename CplxT<R>::typ
             const int i = i0 + t;
             if (i0 > r0) load(i < r1 ? i : -1, b, a);
             Z x = i < r1 ? s_b[i] : zero;
-            static_for<0, 16>([&](auto kc) __attribute__((always_inline)) {
-                constexpr int k = decltype(kc)::value;
-                csubmul(x, a[k], row_bcast_z<k>(xv));
+            R sr = R(0), si = R(0);          // minus the products, summed apart from x
+            static_for<0, 4>([&](auto kc) __attribute__((always_inline)) {
+                zbcast_fma4<4 * decltype(kc)::value>(sr, si, -xv.x, -xv.y, xv.y, a);
             });
+            x.x += sr;
+            x.y += si;
             if (i < r1) s_b[i] = x;
         }
         __syncthreads();
