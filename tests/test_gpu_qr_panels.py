@@ -54,3 +54,31 @@ def test_qr_zero_columns_in_panel(dev):
     assert beta[3] == 0 and beta[8] == 0 and got[3, 3] == 0 and got[8, 8] == 0
     R = np.triu(got[:20])
     assert np.abs(R.T @ R - A.T @ A).max() <= 8 * 300 * EPS64 * np.abs(A.T @ A).max()
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("m", [300, 2000, 4000])
+def test_qr_large_entries(dev, dtype, m):
+    """Columns whose sum overflows but whose norm does not: the reflector of a
+    column of ones has entries of 1 / (1 + sqrt(m)).  Scaling the columns by a
+    power of two scales R's columns, so the reference is LAPACK's R of the
+    scaled matrix; bar 64 m eps of the column's size."""
+    npt = np.float64 if dtype == torch.float64 else np.float32
+    eps, big = float(np.finfo(npt).eps), 2.0 * (float(np.finfo(npt).max) / m)
+    down = 2.0 ** -60
+    A = rng.uniform_matrix(SEED + m, m, 3)
+    A[:, 0] = 1.0
+    A[:, 1] = big * (0.75 + 0.25 * A[:, 1])
+    A[:, 2] *= big
+    A = A.astype(npt)
+    print(f"qr large {dtype} m {m}", flush=True)
+    QR = tmv_amd.colmajor(torch.from_numpy(A).cuda())
+    beta = tmv_amd.geqrf(QR).cpu().numpy()
+    got = QR.cpu().numpy().astype(np.float64)
+    A = A.astype(np.float64)
+    A[:, 1:] *= down
+    (qr, tau), _ = scipy.linalg.qr(A, mode="raw")
+    got[:, 1:][np.triu_indices(m, -1, 2)] *= down       # R's columns, not the reflectors
+    R = np.triu(got[:3])
+    assert np.all(np.abs(R - np.triu(qr[:3])).max(axis=0) <= 64 * m * eps * np.abs(A).max(axis=0))
+    assert np.abs(beta - tau).max() <= 64 * m * eps

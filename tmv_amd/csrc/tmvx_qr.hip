@@ -355,8 +355,22 @@ qr8_panel_kernel(int m, int jb, T* __restrict__ A, i64 lda, T* __restrict__ beta
         const T b = (v0 * v0) / (normsq - y * x0s);
         const T rv0 = T(1) / v0, sinv = rv0 * invscale;
         // dot products with v: lane c that of column c (later column or earlier
-        // reflector), v(k) = 1
-        const T dot = fma(tot, rv0, pv);
+        // reflector), v(k) = 1.  The sums are those of v v0, up to sqrt(m) times
+        // larger: where one overflows, all are formed again with v.
+        T dot = fma(tot, rv0, pv);
+        if (__builtin_amdgcn_ballot_w64(!(tot - tot == T(0)))) {          // uniform
+            T again[8];
+            static_for<0, 8>([&](auto cc) __attribute__((always_inline)) {
+                constexpr int c = decltype(cc)::value;
+                again[c] = T(0);
+                static_for<0, RPT>([&](auto q_) __attribute__((always_inline)) {
+                    constexpr int q = decltype(q_)::value;
+                    const T vr = (q > 0 || t > k) ? row[q][k] * sinv : T(0);
+                    again[c] = fma(vr, row[q][c], again[c]);
+                });
+            });
+            dot = group_sum8(again, s_sum[par ^ 1]) + pv;
+        }
         const T w = b * dot;
         static_for<0, RPT>([&](auto q_) __attribute__((always_inline)) {
             constexpr int q = decltype(q_)::value;
