@@ -82,3 +82,29 @@ def test_qr_large_entries(dev, dtype, m):
     R = np.triu(got[:3])
     assert np.all(np.abs(R - np.triu(qr[:3])).max(axis=0) <= 64 * m * eps * np.abs(A).max(axis=0))
     assert np.abs(beta - tau).max() <= 64 * m * eps
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_qr_finished_rows_take_no_part(dev, dtype):
+    """Q^T b whose first entry overflows (|b| is beyond the largest number,
+    its entries are not): the panels that come later do not see it, and the
+    other unknowns are those of b / 4, times 4."""
+    npt = np.float64 if dtype == torch.float64 else np.float32
+    eps, top = float(np.finfo(npt).eps), float(np.finfo(npt).max)
+    m, n = 64, 16
+    A = 0.1 * rng.uniform_matrix(SEED + 77, m, n)
+    A[:, 0] = 1.0
+    A[0, 0] = 1e-3                 # v = (1, 1/sqrt(63), ..): y0 = -sum(b_r) / sqrt(63)
+    b = np.full((m, 1), 1.12 * (top / (m - 1)) * np.sqrt(m - 1))
+    b[0] = -0.55 * top
+    A, b = A.astype(npt), b.astype(npt)
+    print(f"qr overflow {dtype}", flush=True)
+    QR = tmv_amd.colmajor(torch.from_numpy(A).cuda())
+    beta = tmv_amd.geqrf(QR)
+    small = tmv_amd.colmajor(torch.from_numpy(b / 4).cuda())
+    X = tmv_amd.colmajor(torch.from_numpy(b).cuda())
+    tmv_amd.geqrs(QR, beta, small)
+    tmv_amd.geqrs(QR, beta, X)
+    x, ref = X.cpu().numpy()[1:] / 4, small.cpu().numpy()[1:]
+    assert not np.isfinite(X[0].item()) and np.isfinite(small[0].item())
+    assert np.abs(x - ref).max() <= 64 * m * eps * np.abs(ref).max()

@@ -549,9 +549,11 @@ qr8_form_t_kernel(i64 m, i64 n, const T* __restrict__ QR, i64 lda, const T* __re
 }
 
 // B(:, blockIdx.x) := Q^T B(:, blockIdx.x): the panels in turn, the column in
-// registers, row t + q QN_NTH in thread t's slot q.
+// registers, row t + q QN_NTH in thread t's slot q.  (FP32 with four rows a
+// thread needs a few registers less than it takes for three workgroups a CU.)
 template <typename T, int RPT>
 __global__ void __launch_bounds__(QN_NTH)
+    __attribute__((amdgpu_waves_per_eu(sizeof(T) * RPT <= 16 ? 6 : sizeof(T) * RPT <= 32 ? 4 : 2)))
 qr8_apply_kernel(int m, int n, const T* __restrict__ QR, i64 lda, const T* __restrict__ Tm,
                  T* __restrict__ B, i64 ldb)
 {
@@ -599,11 +601,21 @@ qr8_apply_kernel(int m, int n, const T* __restrict__ QR, i64 lda, const T* __res
                 x[decltype(q_)::value] = fma(-v[decltype(q_)::value][k], zk, x[decltype(q_)::value]);
             });
         });
+        // the panel's own rows are finished: zeros in their place, as an Inf
+        // would reach the others through its zero in V
+        static_for<0, RPT>([&](auto q_) __attribute__((always_inline)) {
+            constexpr int q = decltype(q_)::value;
+            const int r = t + q * QN_NTH;
+            if ((unsigned)(r - j0) < (unsigned)jb) {
+                b[r] = x[q];
+                x[q] = T(0);
+            }
+        });
     }
     static_for<0, RPT>([&](auto q_) __attribute__((always_inline)) {
         constexpr int q = decltype(q_)::value;
         const int r = t + q * QN_NTH;
-        if (r < m) b[r] = x[q];
+        if (r >= n && r < m) b[r] = x[q];
     });
 }
 
