@@ -212,7 +212,7 @@ template <int C, typename Z> __device__ __forceinline__ Z row_bcast_z(Z v)
 #define ZN_FMAC4(SUF, A, B, C, D)                                                            \
     __asm__ volatile("s_nop 1\n\t" ZN_STEP(SUF, A, "%5", "%9") ZN_STEP(SUF, B, "%6", "%10")   \
                          ZN_STEP(SUF, C, "%7", "%11") ZN_STEP(SUF, D, "%8", "%12")           \
-                     : "+v"(xr), "+v"(xi)                                                    \
+                     : "+&v"(xr), "+&v"(xi)                                                    \
                      : "v"(nux), "v"(nuy), "v"(uy), "v"(l[K0].x), "v"(l[K0 + 1].x),          \
                        "v"(l[K0 + 2].x), "v"(l[K0 + 3].x), "v"(l[K0].y), "v"(l[K0 + 1].y),   \
                        "v"(l[K0 + 2].y), "v"(l[K0 + 3].y))

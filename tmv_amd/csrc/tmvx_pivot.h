@@ -118,7 +118,8 @@ __device__ __forceinline__ float row_bcast(float v)
 // compiler does not form by itself; as moves and multiply-adds apart, they
 // also get apart, and the moves' results spill).  Call with every lane active.
 // The leading s_nop: a DPP operand is not read within two wait states of the
-// vector instruction that wrote it.
+// vector instruction that wrote it.  Early-clobber results: the first is
+// written while u and l are still to be read.
 #define TMVX_FMAC8(SUF, A, B, C, D, E, F, G, I)                                                 \
     __asm__ volatile("s_nop 1\n\t"                                                              \
                      "v_fmac_" SUF "_dpp %0, %8, %9 row_newbcast:" A " row_mask:0xf bank_mask:0xf\n\t" \
@@ -129,8 +130,8 @@ __device__ __forceinline__ float row_bcast(float v)
                      "v_fmac_" SUF "_dpp %5, %8, %9 row_newbcast:" F " row_mask:0xf bank_mask:0xf\n\t" \
                      "v_fmac_" SUF "_dpp %6, %8, %9 row_newbcast:" G " row_mask:0xf bank_mask:0xf\n\t" \
                      "v_fmac_" SUF "_dpp %7, %8, %9 row_newbcast:" I " row_mask:0xf bank_mask:0xf"   \
-                     : "+v"(r[C0]), "+v"(r[C0 + 1]), "+v"(r[C0 + 2]), "+v"(r[C0 + 3]),              \
-                       "+v"(r[C0 + 4]), "+v"(r[C0 + 5]), "+v"(r[C0 + 6]), "+v"(r[C0 + 7])          \
+                     : "+&v"(r[C0]), "+&v"(r[C0 + 1]), "+&v"(r[C0 + 2]), "+&v"(r[C0 + 3]),              \
+                       "+&v"(r[C0 + 4]), "+&v"(r[C0 + 5]), "+&v"(r[C0 + 6]), "+&v"(r[C0 + 7])          \
                      : "v"(u), "v"(l))
 template <int H, int C0, int N, typename T>
 __device__ __forceinline__ void bcast_fma8(T (&r)[N], T u, T l)
