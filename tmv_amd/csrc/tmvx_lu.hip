@@ -455,6 +455,9 @@ panel_kernel(T* __restrict__ A, i64 lda, i64 n, i64 j0, int jb, i64* __restrict_
         if (!alive) break;
         if (c0 + BB >= jb) break;
         // -- block end: the BB pivot rows, U12, rank-BB update ---------------
+        // (without the exchange the last column's deferred chunk, if there is
+        // one, reads s_rows after that column's only barrier)
+        if constexpr (SOLO && NBLK - 2 >= BB) __syncthreads();
         if (mypiv >= 0) {
             s_own[mypiv] = 1;
             typedef typename Vec16<T>::type VT;
