@@ -43,7 +43,9 @@ int tmvx_batch_plan_destroy(tmvx_batch_plan plan);
 const char* tmvx_batch_plan_describe(tmvx_batch_plan plan);
 /* Force a schedule: index < tmvx_batch_schedule_count(), wave split,
  * workgroups per CU (1..16).  For tuning experiments and tests: every choice
- * gives the same results. */
+ * gives the same results.  TMVX_ERR_UNSUPPORTED, the plan unchanged, when a
+ * system of n <= split (at most the schedule's 16, 32 or 64) has more than 8
+ * right-hand sides. */
 int tmvx_batch_plan_set(tmvx_batch_plan plan, int schedule, int split, int wgs_per_cu,
                         void* stream);
 int tmvx_batch_schedule_count(void);

@@ -710,6 +710,7 @@ static const BatchKernelInfo kBatchKernels[] = {
 constexpr int kNumBatchKernels = sizeof(kBatchKernels) / sizeof(kBatchKernels[0]);
 // The grid is the work list, a workgroup per system, largest first, so that it
 // balances itself; workgroups per CU are recorded too.
+constexpr int kWaveRhsMax = 8;      // right-hand sides a forced split admits per wave
 constexpr int kBatchSchedule = 2, kBatchSplit = 64, kBatchWgsPerCu = 16;
 
 } // namespace tmvx
@@ -984,6 +985,9 @@ int tmvx_batch_plan_set(tmvx_batch_plan p, int schedule, int split, int wgs_per_
     if (!p || schedule < 0 || schedule >= kNumBatchKernels || split < 0 || wgs_per_cu < 1 ||
         wgs_per_cu > 16)
         return TMVX_ERR_ARG;
+    const int sp = std::min(split, kBatchKernels[schedule].split_max);
+    for (int64_t i = 0; i < p->count; ++i)
+        if (p->h_n[i] <= sp && p->h_nrhs[i] > kWaveRhsMax) return TMVX_ERR_UNSUPPORTED;
     p->tuned_ms = -1.0;
     return plan_build(p, schedule, split, wgs_per_cu, (hipStream_t)stream);
 }
