@@ -27,7 +27,7 @@ Also measured in the same run (outside the K timed steps):
     the CPU-sized case: DGEMM 512^3 and the LU solve n = 512 (A + n I);
   - the batched workload: 20,000 systems n ~ U{8..128} (+ n on the
     diagonal), nrhs ~ U{1..4}, FP64 and FP32, factor + solve in one
-    hipGraph-replayed persistent launch (autotuned plan) vs per-matrix
+    hipGraph replay (three launches) vs per-matrix
     launches, plus the batched GEMM with K = n;
   - the differentiation workload: 512 systems n = 256, forward solve and
     the adjoint (grad_b = A^-T g, grad_A = -grad_b x^T) with stored and
@@ -197,8 +197,8 @@ def cpu_configs(cfg2=False, reps=3):
 
 def batched_workload(torch, tmv_amd, dtype, count=20000, reps=5, per_matrix_sample=200):
     """20,000 independent systems, n ~ U{8..128}, entries uniform[-1,1] + n on
-    the diagonal, nrhs ~ U{1..4}: factor + solve in one persistent launch
-    replayed from a hipGraph (autotuned plan), the batched GEMM C_i = A_i B_i
+    the diagonal, nrhs ~ U{1..4}: factor + solve in three launches
+    replayed from a hipGraph, the batched GEMM C_i = A_i B_i
     with K = n_i, and the same systems through per-matrix launches."""
     import numpy as np
     g = np.random.default_rng(SEED + 30)

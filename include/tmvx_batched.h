@@ -31,8 +31,9 @@ typedef struct tmvx_batch_plan_s* tmvx_batch_plan;
  * A plan for a batch of `count` systems of orders n_host[i] (1..128) with
  * nrhs_host[i] (0..16; NULL = 0: factor only) right-hand sides, in FP64 or
  * FP32.  The plan orders the work list (largest systems first): systems of
- * n <= 64 run one per wave, larger ones one per 128-thread workgroup.
- * tune != 0 also times the plan on a synthetic batch of the same sizes.
+ * n <= 64 run one per wave, larger ones one per 128-thread workgroup.  There
+ * is one schedule; tune != 0 times it on a synthetic batch of the same sizes,
+ * for the plan's text.
  * Allocates device memory and synchronises `stream`; not capturable.
  */
 int tmvx_batch_plan_create(int dtype, int64_t count, const int32_t* n_host,
@@ -42,8 +43,8 @@ int tmvx_batch_plan_destroy(tmvx_batch_plan plan);
 /* Text naming the plan's schedule (valid until the plan changes). */
 const char* tmvx_batch_plan_describe(tmvx_batch_plan plan);
 /* Force a schedule: index < tmvx_batch_schedule_count(), wave split,
- * workgroups per CU (1..16).  For tuning experiments and tests: every choice
- * gives the same results.  TMVX_ERR_UNSUPPORTED, the plan unchanged, when a
+ * workgroups per CU (1..16).  Kept for callers that name one: the choice is
+ * checked and told in the plan's text, and changes nothing else.  TMVX_ERR_UNSUPPORTED, the plan unchanged, when a
  * system of n <= split (at most the schedule's 16, 32 or 64) has more than 8
  * right-hand sides. */
 int tmvx_batch_plan_set(tmvx_batch_plan plan, int schedule, int split, int wgs_per_cu,

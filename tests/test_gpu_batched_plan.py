@@ -22,3 +22,37 @@ def test_forced_schedule_refuses_wide_rhs_per_wave(dev, schedule, cap):
     plan.set(schedule, cap - 1, 2)
     tmv_amd.BatchPlan([cap, 100], [8, 16]).set(schedule, 64, 2)
     tmv_amd.BatchPlan([cap + 1, 100], [9, 16]).set(schedule, cap, 2)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_result_does_not_depend_on_the_batch(dev, dtype):
+    """Bit for bit the same factors, interchanges and solutions by itself, in
+    a batch of its like and among others in another order, with orders on both
+    sides of 32 and 64."""
+    ns = [1, 8, 31, 32, 33, 48, 63, 64, 65, 100, 127, 128]
+    nr = [1, 2, 4, 1, 9, 3, 1, 16, 1, 5, 16, 2]
+    g = np.random.default_rng(3)
+    mats = [torch.from_numpy(g.uniform(-1, 1, (n, n))).to(dtype) for n in ns]
+    rhs = [torch.from_numpy(g.uniform(-1, 1, (n, r))).to(dtype) for n, r in zip(ns, nr)]
+
+    def run(which, fill):
+        idx = list(which)
+        b = tmv_amd.Batch([ns[i] for i in idx] + fill, [nr[i] for i in idx] + [1] * len(fill),
+                          dtype=dtype)
+        b.A.fill_(1.0)
+        for k, i in enumerate(idx):
+            b.a(k).copy_(mats[i])
+            b.b(k).copy_(rhs[i])
+        tmv_amd.gesv_batched(tmv_amd.BatchPlan(b), b)
+        return {i: (b.a(k).cpu(), b.piv(k).cpu(), b.b(k).cpu(), b.info[k].item())
+                for k, i in enumerate(idx)}
+
+    print(f"batch independence {dtype}", flush=True)
+    every = run(range(len(ns)), [])
+    among = run(reversed(range(len(ns))), [1 + 7 * i % 128 for i in range(300)])
+    for i in range(len(ns)):
+        alone = run([i], [])[i]
+        for other in (every[i], among[i]):
+            assert alone[3] == other[3] == 0
+            for u, v in zip(alone[:3], other[:3]):
+                assert torch.equal(u, v), ns[i]

@@ -761,7 +761,7 @@ class Batch:
 
 
 class BatchPlan:
-    """tmvx_batch_plan: the work list and schedule of one batch shape."""
+    """tmvx_batch_plan: the work list of one batch shape."""
 
     def __init__(self, batch_or_ns, nrhs=None, dtype=None, tune=False, stream=None):
         torch = _torch()
@@ -807,7 +807,7 @@ def batch_schedule_count() -> int:
 
 def gesv_batched(plan: BatchPlan, batch: Batch, stream=None):
     """Factor every A_i in place and solve A_i X_i = B_i (B overwritten), in
-    one launch.  Returns the per-system info tensor (device)."""
+    up to three launches.  Returns the per-system info tensor (device)."""
     fn = getattr(lib(), "tmvx_gesv_batched_" + _suffix(batch.dtype))
     _check(fn(plan.handle, batch.pA.data_ptr(), batch.pP.data_ptr(), batch.pB.data_ptr(),
               batch.info.data_ptr(), _stream(stream)), "gesv_batched")

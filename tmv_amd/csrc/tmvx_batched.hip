@@ -4,7 +4,7 @@
 // Counterpart, per system, of TMV's LU_Decompose + LU_LDivEq
 // (src/TMV_LUDecompose.cpp:217-407, src/TMV_LUDiv.cpp:185-226) and MultMM
 // (src/TMV_MultMM.cpp:404-477); TMV has no batched entry point, a caller
-// loops over systems.  Here one persistent launch walks a work list.
+// loops over systems.  Here up to three launches, a workgroup or wave per system.
 //
 // Factor + solve kernels; a system of n <= 64 takes one wave, a larger one
 // (n <= 128) a workgroup of two:
@@ -688,81 +688,64 @@ batched_gemm_kernel(int count, int grp, const int* __restrict__ mv, const int* _
 static int batched_gemm_group(int64_t count) { return count >= 8192 ? 4 : 1; }
 
 // ---------------------------------------------------------------------------
-// Host side: schedule table, plans, autotuning.
+// Host side: plans.
 // ---------------------------------------------------------------------------
-struct BatchKernelInfo {
-    const char* name;
-    int split_max;
-};
 
-// Schedules: every one runs systems of n <= 64 a wave each (what a wave's
-// registers hold) and larger ones a workgroup each; the split and the
-// workgroups per CU that a caller forces are recorded.  Measured, 20,000
-// systems of 8..128 with 1-4 right-hand sides, FP64: 6.80 ms with a 16 x 16
-// thread grid per system and two barriers a column -> 2.05 ms (n > 64 1.80,
-// n <= 64 0.20, n <= 32 0.05); 10,000 of n = 64 3.09 -> 0.29 ms (FP32 2.85 ->
-// 0.15), of n = 32 0.25 -> 0.10, of n = 128 6.24 -> 1.88.
-static const BatchKernelInfo kBatchKernels[] = {
-    {"wave n<=64 (split cap 16) + workgroup n<=128", 16},
-    {"wave n<=64 (split cap 32) + workgroup n<=128", 32},
-    {"wave n<=64 + workgroup n<=128", 64},
-};
-constexpr int kNumBatchKernels = sizeof(kBatchKernels) / sizeof(kBatchKernels[0]);
-// The grid is the work list, a workgroup per system, largest first, so that it
-// balances itself; workgroups per CU are recorded too.
+// One way of running a batch is left, a wave per system of n <= 64 (what a
+// wave's registers hold) and a workgroup per larger one; the grid is the work
+// list, largest first, so that it balances itself.  Measured, 20,000 systems
+// of 8..128 with 1-4 right-hand sides, FP64: 6.80 ms with a 16 x 16 thread
+// grid per system and two barriers a column -> 2.05 ms (n > 64 1.80, n <= 64
+// 0.20, n <= 32 0.05); 10,000 of n = 64 3.09 -> 0.29 ms (FP32 2.85 -> 0.15),
+// of n = 32 0.25 -> 0.10, of n = 128 6.24 -> 1.88.  A schedule that a caller
+// forces (one of three, by the largest order that it gave to a wave) is
+// checked and recorded, and changes nothing else.
+constexpr int kSplitMax[] = {16, 32, 64};
+constexpr int kNumSchedules = 3;
 constexpr int kWaveRhsMax = 8;      // right-hand sides a forced split admits per wave
-constexpr int kBatchSchedule = 2, kBatchSplit = 64, kBatchWgsPerCu = 16;
 
 } // namespace tmvx
 
 struct tmvx_batch_plan_s {
     int dtype = 0;
     int64_t count = 0;
-    int kid = tmvx::kBatchSchedule;
-    int split = tmvx::kBatchSplit;
-    int wgs_per_cu = tmvx::kBatchWgsPerCu;
     int ngroup = 0, nwave64 = 0;        // systems of a workgroup; of a wave, n > 32
-    int cus = 256;
     std::vector<int> h_n, h_nrhs;
     int* d_n = nullptr;
     int4* d_slots = nullptr;
-    double tuned_ms = -1.0;
     char desc[256] = {0};
 };
 
 namespace tmvx {
 
+// The plan's text, with what was timed or forced.
+static void plan_text(tmvx_batch_plan_s* p, const char* more)
+{
+    snprintf(p->desc, sizeof(p->desc), "n<=64 a wave, n<=128 a workgroup: %d + %d + %d systems%s",
+             p->ngroup, p->nwave64, (int)p->count - p->ngroup - p->nwave64, more);
+}
+
 // Build the work list, largest first: systems with n <= 64 take a wave each,
 // the rest a workgroup each.
-static int plan_build(tmvx_batch_plan_s* p, int kid, int split, int wgs_per_cu, hipStream_t s)
+static int plan_build(tmvx_batch_plan_s* p, hipStream_t s)
 {
-    const BatchKernelInfo& K = kBatchKernels[kid];
-    if (split > K.split_max) split = K.split_max;
     const int64_t cnt = p->count;
     std::vector<int> order((size_t)cnt);
     std::iota(order.begin(), order.end(), 0);
     std::stable_sort(order.begin(), order.end(),
                      [&](int a, int b) { return p->h_n[a] > p->h_n[b]; });
     std::vector<int4> slots((size_t)cnt);
-    int ngroup = 0, nwave64 = 0;
     for (int64_t i = 0; i < cnt; ++i) {
         const int k = order[i], n = p->h_n[k];
         slots[i] = int4{k, n, p->h_nrhs[k], 0};
-        if (n > 64) ++ngroup;
-        else if (n > 32) ++nwave64;
+        if (n > 64) ++p->ngroup;
+        else if (n > 32) ++p->nwave64;
     }
-    p->kid = kid;
-    p->split = split;
-    p->wgs_per_cu = wgs_per_cu;
-    p->ngroup = ngroup;
-    p->nwave64 = nwave64;
     if (cnt > 0)
         TMVX_HIP(hipMemcpyAsync(p->d_slots, slots.data(), sizeof(int4) * (size_t)cnt,
                                 hipMemcpyHostToDevice, s));
     TMVX_HIP(hipStreamSynchronize(s));
-    snprintf(p->desc, sizeof(p->desc), "%s; split n<=%d per wave; %d + %d + %d systems; %d/CU%s",
-             K.name, split, ngroup, nwave64, (int)cnt - ngroup - nwave64, wgs_per_cu,
-             p->tuned_ms >= 0 ? "; autotuned" : "");
+    plan_text(p, "");
     return TMVX_OK;
 }
 
@@ -794,7 +777,7 @@ static int batch_launch(const tmvx_batch_plan_s* p, T* const* A, i64* const* piv
 }
 
 // Synthetic batch of the plan's shape (uniform[-1,1] + n I, B uniform) for
-// timing candidate schedules.
+// timing the plan.
 __global__ void batch_diag_shift_kernel(int count, const int* nv, double* const* A64,
                                         float* const* A32)
 {
@@ -812,7 +795,7 @@ __global__ void f64_to_f32_kernel(i64 cnt, const double* in, float* out)
     if (i < cnt) out[i] = (float)in[i];
 }
 
-static int plan_tune(tmvx_batch_plan_s* p, hipStream_t s)
+static int plan_time(tmvx_batch_plan_s* p, hipStream_t s)
 {
     const int64_t cnt = p->count;
     std::vector<i64> offA((size_t)cnt), offB((size_t)cnt), offP((size_t)cnt);
@@ -873,43 +856,35 @@ static int plan_tune(tmvx_batch_plan_s* p, hipStream_t s)
                            p->dtype == 1 ? (float* const*)(dptr + 3 * cnt) : nullptr);
         rc = hip_status(hipGetLastError());
     }
-    // Candidates: one schedule is left to time.
-    struct Cand { int kid, split, wpc; };
-    const std::vector<Cand> cands = {{kBatchSchedule, kBatchSplit, kBatchWgsPerCu}};
-    double best = 1e30;
-    Cand bestc = {p->kid, p->split, p->wgs_per_cu};
-    for (size_t ci = 0; ci < cands.size() && rc == TMVX_OK; ++ci) {
-        const Cand& c = cands[ci];
-        if ((rc = plan_build(p, c.kid, c.split, c.wpc, s)) != TMVX_OK) break;
-        float msbest = 1e30f;
-        for (int rep = 0; rep < 3 && rc == TMVX_OK; ++rep) {   // rep 0 warms up
-            if (hipMemcpyAsync(dA, dA0, esz * ta, hipMemcpyDeviceToDevice, s) != hipSuccess ||
-                hipMemcpyAsync(dB, dB0, esz * tb, hipMemcpyDeviceToDevice, s) != hipSuccess) {
-                rc = TMVX_ERR_HIP;
-                break;
-            }
-            hipEventRecord(e0, s);
-            if (p->dtype == 0)
-                rc = batch_launch<double>(p, (double* const*)dptr, (i64* const*)(dptr + 2 * cnt),
-                                          (double* const*)(dptr + cnt), dinfo, s);
-            else
-                rc = batch_launch<float>(p, (float* const*)dptr, (i64* const*)(dptr + 2 * cnt),
-                                         (float* const*)(dptr + cnt), dinfo, s);
-            hipEventRecord(e1, s);
-            if (hipEventSynchronize(e1) != hipSuccess) { rc = TMVX_ERR_HIP; break; }
-            float ms = 0;
-            hipEventElapsedTime(&ms, e0, e1);
-            if (rep > 0) msbest = std::min(msbest, ms);
+    float best = 1e30f;
+    for (int rep = 0; rep < 3 && rc == TMVX_OK; ++rep) {       // rep 0 warms up
+        if (hipMemcpyAsync(dA, dA0, esz * ta, hipMemcpyDeviceToDevice, s) != hipSuccess ||
+            hipMemcpyAsync(dB, dB0, esz * tb, hipMemcpyDeviceToDevice, s) != hipSuccess) {
+            rc = TMVX_ERR_HIP;
+            break;
         }
-        if (msbest < best) { best = msbest; bestc = c; }
+        hipEventRecord(e0, s);
+        if (p->dtype == 0)
+            rc = batch_launch<double>(p, (double* const*)dptr, (i64* const*)(dptr + 2 * cnt),
+                                      (double* const*)(dptr + cnt), dinfo, s);
+        else
+            rc = batch_launch<float>(p, (float* const*)dptr, (i64* const*)(dptr + 2 * cnt),
+                                     (float* const*)(dptr + cnt), dinfo, s);
+        hipEventRecord(e1, s);
+        if (hipEventSynchronize(e1) != hipSuccess) { rc = TMVX_ERR_HIP; break; }
+        float ms = 0;
+        hipEventElapsedTime(&ms, e0, e1);
+        if (rep > 0) best = std::min(best, ms);
     }
     if (e0) hipEventDestroy(e0);
     if (e1) hipEventDestroy(e1);
     hipFree(dA0); hipFree(dA); hipFree(dB0); hipFree(dB); hipFree(dP); hipFree(dptr);
     hipFree(dinfo); hipFree(stage);
     if (rc != TMVX_OK) return rc;
-    p->tuned_ms = best;
-    return plan_build(p, bestc.kid, bestc.split, bestc.wpc, s);
+    char more[64];
+    snprintf(more, sizeof(more), "; autotuned (one schedule): %.3f ms", best);
+    plan_text(p, more);
+    return TMVX_OK;
 }
 
 } // namespace tmvx
@@ -943,10 +918,6 @@ int tmvx_batch_plan_create(int dtype, int64_t count, const int32_t* n_host,
     p->h_n.assign(n_host, n_host + count);
     p->h_nrhs.assign((size_t)count, 0);
     if (nrhs_host) p->h_nrhs.assign(nrhs_host, nrhs_host + count);
-    int dev = 0;
-    hipDeviceProp_t prop;
-    if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess)
-        p->cus = prop.multiProcessorCount;
     const size_t c1 = (size_t)std::max<int64_t>(count, 1);
     int rc = TMVX_OK;
     if (hipMalloc((void**)&p->d_n, sizeof(int) * c1) != hipSuccess ||
@@ -956,8 +927,8 @@ int tmvx_batch_plan_create(int dtype, int64_t count, const int32_t* n_host,
         hipMemcpyAsync(p->d_n, p->h_n.data(), sizeof(int) * count, hipMemcpyHostToDevice, s) !=
             hipSuccess)
         rc = TMVX_ERR_HIP;
-    if (rc == TMVX_OK) rc = plan_build(p, kBatchSchedule, kBatchSplit, kBatchWgsPerCu, s);
-    if (rc == TMVX_OK && tune && count > 0) rc = plan_tune(p, s);
+    if (rc == TMVX_OK) rc = plan_build(p, s);
+    if (rc == TMVX_OK && tune && count > 0) rc = plan_time(p, s);
     if (rc != TMVX_OK) {
         tmvx_batch_plan_destroy(p);
         return rc;
@@ -980,19 +951,22 @@ const char* tmvx_batch_plan_describe(tmvx_batch_plan p)
     return p ? p->desc : "";
 }
 
-int tmvx_batch_plan_set(tmvx_batch_plan p, int schedule, int split, int wgs_per_cu, void* stream)
+int tmvx_batch_plan_set(tmvx_batch_plan p, int schedule, int split, int wgs_per_cu, void*)
 {
-    if (!p || schedule < 0 || schedule >= kNumBatchKernels || split < 0 || wgs_per_cu < 1 ||
+    if (!p || schedule < 0 || schedule >= kNumSchedules || split < 0 || wgs_per_cu < 1 ||
         wgs_per_cu > 16)
         return TMVX_ERR_ARG;
-    const int sp = std::min(split, kBatchKernels[schedule].split_max);
+    const int sp = std::min(split, kSplitMax[schedule]);
     for (int64_t i = 0; i < p->count; ++i)
         if (p->h_n[i] <= sp && p->h_nrhs[i] > kWaveRhsMax) return TMVX_ERR_UNSUPPORTED;
-    p->tuned_ms = -1.0;
-    return plan_build(p, schedule, split, wgs_per_cu, (hipStream_t)stream);
+    char more[80];
+    snprintf(more, sizeof(more), "; forced (no effect): schedule %d, split %d, %d/CU", schedule, sp,
+             wgs_per_cu);
+    plan_text(p, more);
+    return TMVX_OK;
 }
 
-int tmvx_batch_schedule_count(void) { return kNumBatchKernels; }
+int tmvx_batch_schedule_count(void) { return kNumSchedules; }
 
 int tmvx_gesv_batched_f64(tmvx_batch_plan p, double* const* A, int64_t* const* piv,
                           double* const* B, int32_t* info, void* stream)
