@@ -37,3 +37,11 @@ def test_gemm_batched_groups(dt, count):
                    for v in (av.double(), bv.double(), out))
         bar = (n + 2) * eps * (A.abs() @ B.abs())
         assert bool(((C - A @ B).abs() <= bar).all()), n
+
+
+@pytest.mark.parametrize("dt,count", [(torch.float64, 2047), (torch.float64, 2048),
+                                      (torch.float64, 2051), (torch.float32, 4095),
+                                      (torch.float32, 4096), (torch.float32, 4099)])
+def test_gemm_batched_where_groups_begin(dt, count):
+    """Four problems a workgroup from 2048 (FP64) or 4096 (FP32) on."""
+    test_gemm_batched_groups(dt, count)

@@ -679,13 +679,21 @@ batched_gemm_kernel(int count, int grp, const int* __restrict__ mv, const int* _
     }
 }
 
-// Problems a workgroup: with enough of them to fill the chip several times,
-// four, so that problems of one block (n <= 32) leave no wave idle (20,000 of
-// n = 8, FP64: 33 us against 51 with one); with few, one, so that the larger ones
-// still spread over the CUs (200 of n = 128).
+// Problems a workgroup: with enough of them to fill the chip, four, so that
+// problems of one block (n <= 32) leave no wave idle; with fewer, one, so that
+// the larger ones still spread over the CUs.  One a workgroup -> four (us):
+//   FP64: 8191 of n = 1 27 -> 14, of n = 16 32 -> 18, of n = 32 46 -> 38;
+//         4000 of n = 8 15 -> 10, of n = 128 500 -> 497; 2048 of n = 1 10.0 ->
+//         9.6, of n = 100 218 -> 220; 1500 of n = 128 201 -> 244
+//   FP32 (three workgroups a CU, not two): 8191 of n = 1 14 -> 10, of n = 128
+//         565 -> 579; 6000 of n = 8 12.4 -> 9.8; 3000 of n = 8 8.5 -> 8.3, of
+//         n = 100 197 -> 206
 // Measured, one workgroup a problem with entry loads before: 20,000 of 8..128
-// FP32 1.73 -> 0.82 ms; 4000 of n = 128 FP64 726 -> 506 us, FP32 607 -> 288.
-static int batched_gemm_group(int64_t count) { return count >= 8192 ? 4 : 1; }
+// FP32 1.73 -> 0.82 ms; 4000 of n = 128 FP64 722 -> 497 us, FP32 615 -> 286.
+template <typename T> static int batched_gemm_group(int64_t count)
+{
+    return count >= (sizeof(T) == 8 ? 2048 : 4096) ? 4 : 1;
+}
 
 // ---------------------------------------------------------------------------
 // Host side: plans.
@@ -1026,7 +1034,7 @@ int tmvx_gemm_batched_f64(int64_t count, const int32_t* m, const int32_t* n, con
     if (count < 0 || count > INT_MAX) return TMVX_ERR_ARG;
     if (count == 0) return TMVX_OK;
     if (!m || !n || !k || !A || !B || !C) return TMVX_ERR_ARG;
-    const int grp = batched_gemm_group(count);
+    const int grp = batched_gemm_group<double>(count);
     const unsigned grid = (unsigned)std::min<int64_t>((count + grp - 1) / grp, 1 << 20);
     hipLaunchKernelGGL(batched_gemm_kernel<double>, dim3(grid), dim3(256), 0,
                        (hipStream_t)stream, (int)count, grp, m, n, k, alpha, A, B, beta, C);
@@ -1040,7 +1048,7 @@ int tmvx_gemm_batched_f32(int64_t count, const int32_t* m, const int32_t* n, con
     if (count < 0 || count > INT_MAX) return TMVX_ERR_ARG;
     if (count == 0) return TMVX_OK;
     if (!m || !n || !k || !A || !B || !C) return TMVX_ERR_ARG;
-    const int grp = batched_gemm_group(count);
+    const int grp = batched_gemm_group<float>(count);
     const unsigned grid = (unsigned)std::min<int64_t>((count + grp - 1) / grp, 1 << 20);
     hipLaunchKernelGGL(batched_gemm_kernel<float>, dim3(grid), dim3(256), 0,
                        (hipStream_t)stream, (int)count, grp, m, n, k, alpha, A, B, beta, C);
