@@ -56,3 +56,26 @@ def test_result_does_not_depend_on_the_batch(dev, dtype):
             assert alone[3] == other[3] == 0
             for u, v in zip(alone[:3], other[:3]):
                 assert torch.equal(u, v), ns[i]
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("n", [1, 3, 32, 33, 64])
+def test_columns_do_not_depend_on_their_number(dev, dtype, n):
+    """Right-hand sides go four at a time and a last one by itself: each
+    column is bit for bit that of a solve of its own."""
+    g = np.random.default_rng(n)
+    A = torch.from_numpy(g.uniform(-1, 1, (n, n))).to(dtype)
+    B = torch.from_numpy(g.standard_normal((n, 16))).to(dtype)
+
+    def run(counts):
+        b = tmv_amd.Batch([n] * len(counts), [len(c) for c in counts], dtype=dtype)
+        for k, c in enumerate(counts):
+            b.a(k).copy_(A)
+            b.b(k).copy_(B[:, c])
+        tmv_amd.gesv_batched(tmv_amd.BatchPlan(b), b)
+        return [b.b(k).cpu() for k in range(len(counts))]
+
+    print(f"columns n {n} {dtype}", flush=True)
+    single = torch.cat(run([[c] for c in range(16)]), dim=1)
+    for r, x in zip(range(17), run([list(range(r)) for r in range(17)])):
+        assert torch.equal(x, single[:, :r]), r

@@ -327,7 +327,7 @@ __device__ __forceinline__ void store_row(const T (&row)[N], T* A, i64 ld, int m
 // loop keeps in registers from one to the next is more than there are.)
 template <typename T, int N>
 __global__ void __launch_bounds__(64)
-    __attribute__((amdgpu_waves_per_eu(sizeof(T) * N >= 512 ? 2 : 4)))
+    __attribute__((amdgpu_waves_per_eu(sizeof(T) * N >= 512 ? 2 : sizeof(T) * N >= 256 ? 4 : 5)))
 batched_lu_wave_kernel(BatchArgs<T> args)
 {
     __shared__ PanelLds<T, N, 1> L;
@@ -349,9 +349,13 @@ batched_lu_wave_kernel(BatchArgs<T> args)
     store_row(row, A, (i64)n, n, n, lane, pos);
     for (int k = lane; k < n; k += 64) piv[k] = L.piv[k];
     if (lane == 0) args.info[idx] = first_zero;
-    // (one right-hand side as one column: a quarter of the work)
-    if (nr == 1) solve_rows<1>(row, n, nr, B, (i64)n, lane, pos, rdiag, first_zero != 0);
-    else if (nr > 1) solve_rows<4>(row, n, nr, B, (i64)n, lane, pos, rdiag, first_zero != 0);
+    // (a last right-hand side by itself as one column: a quarter of the work;
+    // one after the other, not one or the other, for which the compiler saved
+    // the rows to memory first, with no right-hand side too)
+    const int nr4 = (nr & 3) == 1 ? nr - 1 : nr;
+    solve_rows<4>(row, n, nr4, B, (i64)n, lane, pos, rdiag, first_zero != 0);
+    if (nr4 < nr)
+        solve_rows<1>(row, n, 1, B + nr4 * (i64)n, (i64)n, lane, pos, rdiag, first_zero != 0);
 }
 
 // System slots[blockIdx.x], 64 < n <= 128, a workgroup of two waves.
