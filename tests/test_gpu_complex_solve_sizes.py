@@ -65,3 +65,41 @@ def test_complex_solve_singular(dev, n):
     x[n // 2] = 1
     with pytest.raises(tmv_amd.TmvxError):
         tmv_amd.getrs_complex(LU, piv, x)
+
+
+@pytest.mark.parametrize("dtype", [torch.complex128, torch.complex64])
+@pytest.mark.parametrize("trans", [False, True])
+@pytest.mark.parametrize("n", [5, 40, 600, 2100, 4097])
+def test_complex_zero_entry_takes_no_part(dev, n, trans, dtype):
+    """A zero entry is skipped by the substitution: Inf and NaN in its column
+    of the factors (or, transposed, its row) do not matter, and a zero on U's
+    diagonal there is not reported.  Same bar as above."""
+    g = np.random.default_rng(n)
+    h = n // 2
+    LU = ((g.uniform(-1, 1, (n, n)) + 1j * g.uniform(-1, 1, (n, n))) * (0.7 / n)).astype(np.complex64)
+    np.fill_diagonal(LU, 1 + g.random(n))
+    B = np.zeros((n, 2), np.complex128)
+    if trans:
+        B[h] = (1, -2j)             # U^T x = b: zero before row h
+        clean = LU.copy()
+        LU[: h, h:] = np.nan
+        LU[0, 0] = 0
+        clean[: h, h:] = 0
+    else:
+        B[h] = (1, -2j)             # L: row h alone; U: nothing below it
+        LU[h + 1:, h] = 0
+        clean = LU.copy()
+        LU[1:, 0] = np.inf
+        LU[: n - 1, n - 1] = np.nan
+        LU[n - 1, n - 1] = 0
+        clean[1:, 0] = clean[: n - 1, n - 1] = 0
+        clean[n - 1, n - 1] = 1
+    L, U = np.tril(clean, -1).astype(np.complex128) + np.eye(n), np.triu(clean).astype(np.complex128)
+    print(f"complex zeros n {n} trans {trans} {dtype}", flush=True)
+    x = tmv_amd.colmajor(torch.from_numpy(B).to(dtype).cuda())
+    tmv_amd.getrs_complex(tmv_amd.colmajor(torch.from_numpy(LU).to(dtype).cuda()),
+                          torch.arange(n, device="cuda"), x, trans=trans)
+    X = x.cpu().numpy().astype(np.complex128)
+    back = L @ (U @ X) if not trans else U.T @ (L.T @ X)
+    part = torch.float64 if dtype == torch.complex128 else torch.float32
+    assert np.abs(back - B).max() <= 6 * n * torch.finfo(part).eps * np.abs(B).max()

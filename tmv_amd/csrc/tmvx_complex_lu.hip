@@ -572,18 +572,17 @@ __global__ void zpermute_kernel(i64 n, i64 nrhs, typename CplxT<R>::type* __rest
     }
 }
 
-// Triangular column sweep on one right-hand side per workgroup.
+// Triangular column sweep on one right-hand side b (memory or LDS) by a
+// workgroup.
 //   mode 0: L x = b (unit lower), forward      mode 1: U x = b (upper), backward
 //   mode 2: U^T x = b (lower), forward         mode 3: L^T x = b (unit upper), backward
 // A zero U diagonal met by a non-zero entry sets *singular.
 template <typename R>
-__global__ void __launch_bounds__(256)
-zsweep_kernel(i64 n, const typename CplxT<R>::type* __restrict__ LU, i64 lda,
-              typename CplxT<R>::type* __restrict__ B, i64 ldb, int mode, int* __restrict__ singular)
+__device__ __forceinline__ void zsweep(i64 n, const typename CplxT<R>::type* __restrict__ LU,
+                                       i64 lda, typename CplxT<R>::type* b, int mode,
+                                       typename CplxT<R>::type& s_x, int* __restrict__ singular)
 {
     typedef typename CplxT<R>::type Z;
-    __shared__ Z s_x;
-    Z* b = B + (i64)blockIdx.x * ldb;
     const int t = threadIdx.x;
     const bool fwd = mode == 0 || mode == 2;
     const bool diag = mode == 1 || mode == 2;
@@ -625,12 +624,21 @@ zsweep_kernel(i64 n, const typename CplxT<R>::type* __restrict__ LU, i64 lda,
     }
 }
 
+template <typename R>
+__global__ void __launch_bounds__(256)
+zsweep_kernel(i64 n, const typename CplxT<R>::type* __restrict__ LU, i64 lda,
+              typename CplxT<R>::type* __restrict__ B, i64 ldb, int mode, int* __restrict__ singular)
+{
+    __shared__ typename CplxT<R>::type s_x;
+    zsweep<R>(n, LU, lda, B + (i64)blockIdx.x * ldb, mode, s_x, singular);
+}
+
 // One right-hand side per workgroup, n <= ZS_NMAX: both triangular solves on
 // the vector in LDS.  Blocks of 16 rows: a thread loads its row's 16 entries of
 // the block's columns, the first wave meanwhile solves the block (a row per
 // lane, solved entries by DPP broadcast, one division an entry), then every row
 // to come takes the block's product.  Bound: the block's chain of 16 divisions
-// and one barrier pair per block.  mode as in zsweep_kernel; perm: row i of P A
+// and one barrier pair per block.  mode as in zsweep; perm: row i of P A
 // is row perm[i] of A.
 constexpr int ZS_NMAX = 4096;
 constexpr int ZS_NTH = 512;
@@ -724,17 +732,34 @@ zsolve_kernel(int trans, int n, const typename CplxT<R>::type* __restrict__ LU, 
 {
     typedef typename CplxT<R>::type Z;
     __shared__ __attribute__((aligned(16))) Z s_b[ZS_NMAX];
+    __shared__ Z s_x;
+    __shared__ int s_sing;
     Z* b = B + (i64)blockIdx.x * ldb;
     const int t = threadIdx.x;
     for (int i = t; i < n; i += ZS_NTH) s_b[i] = trans ? b[i] : b[perm[i]];
+    if (t == 0) s_sing = 0;
     __syncthreads();
     if (!trans) {
-        zsolve_sweep<R, 0>(n, LU, lda, s_b, singular);
-        zsolve_sweep<R, 1>(n, LU, lda, s_b, singular);
+        zsolve_sweep<R, 0>(n, LU, lda, s_b, &s_sing);
+        zsolve_sweep<R, 1>(n, LU, lda, s_b, &s_sing);
     } else {
-        zsolve_sweep<R, 2>(n, LU, lda, s_b, singular);
-        zsolve_sweep<R, 3>(n, LU, lda, s_b, singular);
+        zsolve_sweep<R, 2>(n, LU, lda, s_b, &s_sing);
+        zsolve_sweep<R, 3>(n, LU, lda, s_b, &s_sing);
     }
+    // A zero entry takes no part in a substitution (src/TMV_TriDiv_V.cpp:187),
+    // but a zero times an Inf or NaN of the factors does in a block of 16: a
+    // solution with a NaN is found again by column sweeps, which skip it.
+    int bad = 0;
+    for (int i = t; i < n; i += ZS_NTH) bad |= s_b[i].x != s_b[i].x || s_b[i].y != s_b[i].y;
+    if (__syncthreads_or(bad)) {
+        for (int i = t; i < n; i += ZS_NTH) s_b[i] = trans ? b[i] : b[perm[i]];
+        if (t == 0) s_sing = 0;
+        __syncthreads();
+#pragma clang loop unroll(disable)
+        for (int mode = trans ? 2 : 0; mode < (trans ? 4 : 2); ++mode)
+            zsweep<R>(n, LU, lda, s_b, mode, s_x, &s_sing);
+    }
+    if (t == 0 && s_sing) *singular = 1;
     for (int i = t; i < n; i += ZS_NTH) b[trans ? perm[i] : i] = s_b[i];
 }
 
