@@ -54,3 +54,28 @@ def test_gemm_edges_every_config(dt, layouts, pad, shift):
                 assert rc == 0
                 d = (C.t().double() - ref).abs()
                 assert bool((d <= bar).all()), (cfg, m, n, k)
+
+
+@pytest.mark.parametrize("dt", [torch.float64, torch.float32])
+@pytest.mark.parametrize("layouts", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_gemm_bits_do_not_depend_on_the_tile(dt, layouts):
+    """Every configuration adds an entry's products in the same order, so a
+    factorisation may take another tile beside a panel than alone."""
+    L = tmv_amd.lib()
+    eb = 8 if dt == torch.float64 else 4
+    fn = L.tmvx_gemm_cfg_f64 if eb == 8 else L.tmvx_gemm_cfg_f32
+    la, lb = layouts
+    gen = torch.Generator().manual_seed(6)
+    for m, n, k in ((130, 257, 256), (300, 200, 289), (64, 64, 31), (1100, 1030, 256)):
+        A, lda, _ = operand(m, k, la, 0, 0, dt, gen)
+        B, ldb, _ = operand(k, n, lb, 0, 0, dt, gen)
+        C0 = (torch.rand(n, m, dtype=dt, generator=gen) * 2 - 1).cuda()
+        first = None
+        for cfg in range(L.tmvx_gemm_config_count(eb)):
+            C = C0.clone()
+            rc = fn(cfg, la, lb, m, n, k, -1.0, A.data_ptr(), lda, B.data_ptr(), ldb, 1.0,
+                    C.data_ptr(), m, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+            assert rc == 0
+            if first is None:
+                first = C
+            assert torch.equal(C, first), (cfg, m, n, k)

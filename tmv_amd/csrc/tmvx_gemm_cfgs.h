@@ -1,4 +1,7 @@
 // GEMM tile-configuration tables: X(id, BM, BN, BK, WM, WN, min waves/SIMD).
+// The tile does not show in the result: whatever BM, BN and BK, an entry of C
+// is one MFMA chain over k, 16 at a time, the last ones filled up with zeros.
+// The LU relies on it where it takes another tile beside a panel than alone.
 // Measured on MI355X, column-major operands, beta != 0 (us):
 //                       f64 0    1    2    4 | f32 0    1    2    3    4
 //   512^3                  26   76   41   12 |    47   53   30   17    8

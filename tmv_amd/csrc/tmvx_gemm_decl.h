@@ -13,8 +13,6 @@ struct GemmCfg {
     static constexpr int V = Vec16<T>::n;            // elements per 16 B
     static constexpr int TM = BM / WM, TN = BN / WN; // wave tile
     static constexpr int FM = TM / 16, FN = TN / 16; // MFMA blocks per wave
-    static constexpr int PADK = 16 / sizeof(T);      // pad of k-contiguous rows (16 B)
-    static constexpr int PADX = 16 / sizeof(T);      // pad of k-major rows (16 B)
     static constexpr int NVA = BM * BK / V / NT;     // 16 B loads per thread
     static constexpr int NVB = BN * BK / V / NT;
     // stages in flight: two where several workgroups a CU also cover the

@@ -18,7 +18,8 @@ namespace tmvx {
 //
 // With na != nullptr (no allocation): the workspace is na->ws (at most
 // na->bytes; larger n is TMVX_ERR_UNSUPPORTED), the look-ahead's side work
-// runs on s itself (same kernels, same order, so the same results), and
+// runs on s itself (the same products in the same order; an FP32 update may
+// take another tile, which adds them in the same order: the same results), and
 // nothing is synchronised or copied to the host: na->d_info (device)
 // receives the info, or -1 when a bounded wait expired.  FP32/FP64 partial
 // pivoting only.

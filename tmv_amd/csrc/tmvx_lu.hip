@@ -104,17 +104,6 @@ template <typename T, int BB> struct ColSlot {
 };
 
 template <typename T>
-__device__ __forceinline__ unsigned half_bits(T v, int h)
-{
-    if constexpr (sizeof(T) == 8) {
-        const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-        return h ? (unsigned)(b >> 32) : (unsigned)b;
-    } else {
-        return (unsigned)__float_as_uint(v);
-    }
-}
-
-template <typename T>
 __device__ __forceinline__ T from_halves(const unsigned* h)
 {
     if constexpr (sizeof(T) == 8)
