@@ -108,3 +108,34 @@ def test_qr_finished_rows_take_no_part(dev, dtype):
     x, ref = X.cpu().numpy()[1:] / 4, small.cpu().numpy()[1:]
     assert not np.isfinite(X[0].item()) and np.isfinite(small[0].item())
     assert np.abs(x - ref).max() <= 64 * m * eps * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("dtype,m,n", [
+    (torch.float64, 9, 7), (torch.float64, 513, 64), (torch.float64, 1025, 33),
+    (torch.float64, 4096, 17), (torch.float64, 4097, 12), (torch.float32, 600, 31),
+    (torch.float32, 2100, 16)])
+def test_qr_reproduces_the_matrix(dev, dtype, m, n):
+    """A = Q R to 8 m eps |A|, with Q formed on the host from the reflectors
+    in long double, and the applied Q^T: the solve with A itself on the right
+    gives X with R X = R (R x = y to n eps |R||x| beside) and nothing below."""
+    print(f"qr product {dtype} {m}x{n}", flush=True)
+    eps = EPS64 if dtype == torch.float64 else EPS32
+    A = rng.uniform_matrix(SEED + 5 * m + n, m, n)
+    if dtype == torch.float32:
+        A = A.astype(np.float32).astype(np.float64)
+    QR = tmv_amd.colmajor(torch.from_numpy(A).to(dtype).cuda())
+    beta = tmv_amd.geqrf(QR)
+    got, b = QR.cpu().numpy().astype(np.longdouble), beta.cpu().numpy().astype(np.longdouble)
+    P = np.zeros((m, n), np.longdouble)
+    P[:n] = np.triu(got[:n])
+    for j in range(n - 1, -1, -1):
+        v = np.concatenate([np.ones(1, np.longdouble), got[j + 1:, j]])
+        P[j:] -= np.outer(v, b[j] * (v @ P[j:]))
+    big = np.abs(A).max()
+    assert np.abs(P - A).max() <= 8 * m * eps * big
+    X = tmv_amd.colmajor(torch.from_numpy(A).to(dtype).cuda())
+    tmv_amd.geqrs(QR, beta, X)
+    x, R = X.cpu().numpy().astype(np.longdouble), np.triu(got[:n])
+    bar = 8 * m * eps * big + n * eps * (np.abs(R) @ np.abs(x[:n])).max()
+    assert np.abs(R @ x[:n] - R).max() <= bar
+    assert m == n or np.abs(x[n:]).max() <= 8 * m * eps * big
