@@ -61,11 +61,11 @@ SEED = 0x7A15EED
 # HBM bytes per launch of the 8192^3 CCC DGEMM (gemm_kernel f64 128x128x16),
 # from rocprofv3 --pmc FETCH_SIZE (x2.0) and WRITE_SIZE (x1.0), the factors a
 # 1 GiB device copy reads on the same counters; profiles/dgemm_8192_ccc_traffic.md.
-DGEMM_8192_CCC_TRAFFIC = 13.71e9
+DGEMM_8192_CCC_TRAFFIC = 13.43e9
 # HBM bytes per launch of the FP32 panel kernel (64-column panels), averaged
 # over the 256 panels of an n = 16384 LU (same counters and factors);
 # profiles/panel_f32_n16384_traffic.md.
-PANEL_F32_16384_TRAFFIC = {64: 6.25e6}
+PANEL_F32_16384_TRAFFIC = {64: 6.40e6}
 
 
 def conditioned_gpu(n, kappa, seed, torch, tmv_amd):
