@@ -113,10 +113,10 @@ int tmvx_getrf_batched_f32(int64_t count, const int32_t* n_host, float* const* A
  * factors (LU_i, piv_i), the solutions X_i and the cotangents G_i = dL/dX_i
  * (all n_i x nrhs_i, leading dimension n_i):
  *   gradB_i = A_i^-T G_i,   gradA_i = -gradB_i X_i^T (+ gradA_i if accumulate)
- * One wave per system; the rank-nrhs update is fused into the kernel that
- * solves for gradB_i, so gradA_i is written once.  n, nrhs are device
- * arrays.  One launch, capturable.  No counterpart in TMV (no derivatives);
- * per system the transposed solve is LU_RDivEq (src/TMV_LUDiv.cpp:369-410).
+ * Two launches, capturable: gradB_i by a workgroup per system (n_i <= 64: a
+ * wave; more than 1024 systems: a wave each), then gradA_i by many workgroups
+ * per system, written once.  n, nrhs are device arrays.  No counterpart in
+ * TMV (no derivatives); per system the transposed solve is LU_RDivEq (src/TMV_LUDiv.cpp:369-410).
  */
 int tmvx_gesv_adjoint_batched_f64(int64_t count, const int32_t* n, const int32_t* nrhs,
                                   const double* const* LU, const int64_t* const* piv,

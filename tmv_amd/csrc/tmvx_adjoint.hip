@@ -9,10 +9,10 @@
 // (x % A, src/TMV_LUDiv.cpp:369-410) and the rank-k update its MultMM
 // (src/TMV_MultMM.cpp:404-477).
 //
-// Batched kernels: a workgroup or a wave per system solves A^T gB = G with the stored factors; then many workgroups per system write
-// gradA as
-// -sum_c gB(:,c) X(k,c), 16 columns each (gradA, the n^2 output, is
-// written once and read only when accumulating).  The recompute variant
+// Batched kernels: a workgroup or a wave per system solves A^T gB = G with the
+// stored factors; then many workgroups per system write gradA as
+// -sum_c gB(:,c) X(k,c), 16 columns each (gradA, the n^2 output, is written
+// once and read only when accumulating).  The recompute variant
 // factors copies of the original matrices first, for callers that did not
 // keep the factors.
 #include "tmvx_lu.h"

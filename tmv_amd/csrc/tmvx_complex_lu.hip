@@ -27,10 +27,10 @@
 // Solves up to ZS_NMAX: one workgroup per right-hand side, the vector in LDS,
 // 16 rows at a time (substitution on 16 lanes, then the rows to come with the
 // next 16 columns already loaded); above: column sweeps by one workgroup.
-// Bound: the panel's chain (1.3-1.8 us a column, most of it hypot, the pivot's
+// Bound: the panel's chain (1.4-1.9 us a column, most of it hypot, the pivot's
 // reciprocal and one barrier) and two launches per 16 columns.  Measured at
-// n = 1000, 4 right-hand sides, FP64: 22.1 -> 3.1 ms (panels 12.0 -> 1.6, U12
-// and update 5.8 -> 0.7, solves 2.9 -> 0.6, left interchanges 0.1).
+// n = 1000, 4 right-hand sides, FP64: 22.1 -> 3.3 ms (panels 12.0 -> 1.7, U12
+// and update 5.8 -> 0.8, solves 2.9 -> 0.6, left interchanges 0.1).
 #include "tmvx_lu.h"
 #include "tmvx_pivot.h"
 

@@ -48,7 +48,17 @@ template <> struct GemmTable<float> {
 //     15.7; but 4.2 ms against 3.9 at 5000^3, 10% idle);
 //   - else 128 x 64 where C is large, 64 x 64 below and for a short K:
 //     several workgroups a CU hide each other's waits and the read and write
-//     of C (8192 x 8192 x 128 FP32 278-289 us against 302);
+//     of C (8192 x 8192 x 128 FP32 278-289 us against 302).  The line lies
+//     where 128 x 64 starts to win on some shapes; time of 64 x 64 over that
+//     of 128 x 64, square column-major products, FP64 / FP32:
+//       n     1777  2048         2500         3072         4096
+//             1.06  1.00 / 0.98  0.88 / 0.87  0.90 / 0.91  0.99 / 1.02
+//     and 1.00-1.04 above 16e6 entries.  Which is faster turns on how full
+//     the last turn over the 256 CUs is, and FP32 with a row-major A gains
+//     (3001 x 1777 x 2500: 1.04-1.06) where column-major loses: from the line
+//     to 16e6 entries this costs about 3% (FP64) and 5% (FP32) on average
+//     against the better of the two, and a line at 16e6 would cost 1%, but
+//     4-6% on the shapes named here;
 //   - in FP32 a row-major B takes 128 x 64 in place of 128 x 128 tiles
 //     (4096^3: 1.05 ms against 1.22).
 template <typename T> int default_cfg(int tb, i64 m, i64 n, i64 k)
