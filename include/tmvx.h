@@ -102,7 +102,7 @@ int tmvx_getrf_mn_f32(int64_t m, int64_t n, float* A, int64_t lda, int64_t* piv,
  * tmvx_getrf_f64 that allocates nothing: no counterpart in TMV; for callers
  * that cannot allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc).  The same factorisation
- * (same kernels in the same order: identical pivots and factors) on
+ * (same operations in the same order: identical pivots and factors) on
  * `stream` alone, asynchronous: *d_info (DEVICE int64) receives the 1-based
  * first zero pivot, 0, or -1 when a bounded device-side wait expired; the
  * call neither synchronises nor copies to the host.  Its scratch (panel
